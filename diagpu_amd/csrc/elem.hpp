@@ -44,6 +44,7 @@ __device__ __forceinline__ cf32 scale_(cf32 a, cf32 x)
     return r;
 }
 __device__ __forceinline__ float add_(float a, float b) { return a + b; }
+__device__ __forceinline__ double add_(double a, double b) { return a + b; }
 __device__ __forceinline__ cf32 add_(cf32 a, cf32 b) { return cf32{a.re + b.re, a.im + b.im}; }
 
 __device__ __forceinline__ float sel(bool c, float a, float b) { return c ? a : b; }

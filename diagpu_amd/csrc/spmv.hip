@@ -37,7 +37,9 @@
 // drain anywhere (measured against 64 offsets per VGPR broadcast by
 // readlane, with a refill of that VGPR every 64 diagonals: 1.7 points of
 // 8 TB/s on config 3's 64 diagonals, about 1 point at 85 and 377).  For
-// K <= 5 the short kernel issues all 2K loads straight-line.
+// K <= 16 the short kernel issues all 2K loads straight-line.  Where the rows
+// are too few to fill the chip with waves, several waves share a tile and
+// split its diagonals (spmv_split_kernel).
 //
 // Edge tiles.  A tile whose rows or columns leave the matrix for some
 // diagonal runs the same ring, still with 16-byte runs, each loaded at its
@@ -65,6 +67,7 @@
 // partial; a one-workgroup kernel launched next adds the partials in tile
 // order (a deterministic result).
 #include <climits>
+#include <type_traits>
 
 #include "common.hpp"
 #include "elem.hpp"
@@ -76,6 +79,7 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kShortMax = 16;   // K <= kShortMax: straight-line kernel
+constexpr int kSplitChunk = 8;   // split kernel: diagonals whose loads a wave issues at once
 
 // Per (matrix element, vector element) pair: rows per lane and ring depths,
 // chosen so the kernels stay within 64 VGPRs (8 waves per SIMD).
@@ -379,6 +383,133 @@ __global__ __launch_bounds__(kBlock) void spmv_narrow_kernel(
     if constexpr (DOT) dot_epilogue<TX, R>(acc, x, r, rows, false, tile, tiles, da);
 }
 
+// m diagonals (1 <= m <= N) of an interior tile: all 2 N loads at once, the
+// slots past m a copy of the last diagonal's whose terms are dropped.
+template <typename TV, typename TX, int N>
+__device__ __forceinline__ void straight_chunk(int64_t r, int64_t cols, int m,
+                                               const int32_t* __restrict__ offs,
+                                               const TV* __restrict__ vg,
+                                               const TX* __restrict__ x,
+                                               Run<TX, Shape<TV, TX>::R>& acc)
+{
+    constexpr int R = Shape<TV, TX>::R;
+    Run<TV, R> a[N];
+    Run<TX, R> b[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int k = j < m ? j : m - 1;
+        const int64_t c = r + offs[k];
+        a[j] = load_run<TV, R, true>(vg + (int64_t)k * cols + c);
+        b[j] = load_run<TX, R, false>(x + c);
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int e = 0; e < R; ++e)
+            acc.v[e] = sel(j < m, mad(acc.v[e], a[j].v[e], b[j].v[e]), acc.v[e]);
+}
+
+// Few rows, many diagonals (split_waves): S waves share one tile of 64 R
+// rows, wave w accumulating the diagonals [K w / S, K (w + 1) / S), and the
+// S sums of each row are added in wave order through LDS (a fixed order:
+// deterministic).
+//
+// What bounds such a call is the chain of load latencies of one wave over
+// its K diagonals, with too few waves to hide it (fp64, n = 100003, K = 64:
+// 200 workgroups of the ring kernel on 256 CUs).  S waves per row cut the
+// chain to K / S diagonals, taken in chunks of at most kSplitChunk whose
+// loads are all in flight at once (exact chunk sizes 2, 4, 6, 8: padding
+// slots would be real loads), and put S times as many waves on the chip.
+template <typename TV, typename TX, int S>
+__global__ __launch_bounds__(64 * S) void spmv_split_kernel(
+    int32_t rows, int32_t cols, int64_t lim, int32_t K, const int32_t* __restrict__ offs,
+    const TV* __restrict__ vals, const TX* __restrict__ x, TX* __restrict__ y, int32_t tiles,
+    int32_t per_xcd)
+{
+    constexpr int R = Shape<TV, TX>::R;
+    constexpr int kRows = 64 * R;
+    __shared__ Run<TX, R> part[S * 64];
+    const int tile = tile_of_block(per_xcd);
+    if (tile >= tiles) return;   // uniform over the workgroup
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int64_t r0 = (int64_t)tile * kRows;
+    const int64_t r = r0 + (int64_t)lane * R;
+    // K >= S (split_waves): every wave has a diagonal
+    const int k0 = (int)((int64_t)K * wave / S);
+    const int gn = (int)((int64_t)K * (wave + 1) / S) - k0;
+    const int32_t* od = offs + k0;
+    const TV* vg = vals + (int64_t)k0 * cols;
+
+    int dmin = INT_MAX, dmax = INT_MIN;
+    for (int g0 = 0; g0 < gn; g0 += 64) {
+        const int gm = (gn - g0) < 64 ? (gn - g0) : 64;
+        int lo, hi;
+        wave_minmax(od[g0 + (lane < gm ? lane : gm - 1)], lo, hi);
+        dmin = lo < dmin ? lo : dmin;
+        dmax = hi > dmax ? hi : dmax;
+    }
+    const bool interior =
+        r0 + kRows <= rows && r0 + dmin >= 0 && r0 + kRows + (int64_t)dmax <= lim;
+
+    Run<TX, R> acc;
+#pragma unroll
+    for (int e = 0; e < R; ++e) acc.v[e] = zero_of<TX>();
+    if (!interior) {
+        edge_group<TV, TX>(r, cols, lim, gn, od, vg, x, acc);
+    } else {
+        // equal chunks of at most kSplitChunk diagonals, each chunk's loads
+        // straight-line
+        const int chunks = (gn + kSplitChunk - 1) / kSplitChunk;
+        for (int c = 0; c < chunks; ++c) {
+            const int a0 = (int)((int64_t)gn * c / chunks);
+            const int m = (int)((int64_t)gn * (c + 1) / chunks) - a0;
+            const TV* vc = vg + (int64_t)a0 * cols;
+            if (m > 6)
+                straight_chunk<TV, TX, 8>(r, cols, m, od + a0, vc, x, acc);
+            else if (m > 4)
+                straight_chunk<TV, TX, 6>(r, cols, m, od + a0, vc, x, acc);
+            else if (m > 2)
+                straight_chunk<TV, TX, 4>(r, cols, m, od + a0, vc, x, acc);
+            else
+                straight_chunk<TV, TX, 2>(r, cols, m, od + a0, vc, x, acc);
+        }
+    }
+    part[threadIdx.x] = acc;
+    __syncthreads();
+    // row i of the tile: lane i / R's element i % R of every wave
+    const TX* p = reinterpret_cast<const TX*>(part);
+    for (int i = (int)threadIdx.x; i < kRows; i += 64 * S) {
+        TX sum = p[i];
+#pragma unroll
+        for (int w = 1; w < S; ++w) sum = add_(sum, p[w * kRows + i]);
+        if (r0 + i < rows) y[r0 + i] = sum;
+    }
+}
+
+// Waves per tile of the split kernel, or 1 for the other kernels: a rule on
+// rows and diagonals alone, so that a real matrix takes the same order of
+// sums with real and with complex vectors.  About 8 diagonals per wave (4
+// at K <= 16, where the short kernel already issues every load at once).
+// Measured (us, 3 rotated sets, ring or short kernel -> split):
+//   fp32, K 64:  n = 1000 18.1 -> 5.4, 100003 17.5 -> 6.8, 300007 22.5 ->
+//                14.2, 600011 30.9 -> 26.8, 10^6 43.9 -> 43.7, 2 10^6 89.2
+//                -> 89.6
+//   fp64, K 64:  n = 100003 14.2 -> 11.8, 300007 30.7 -> 27.6, 10^6 88.6 ->
+//                92.3;  complex, K 85, n = 300007: 43.3 -> 41.8
+//   fp32 matrix, complex vector (half the rows per lane, so twice the
+//   waves): K 64, n = 300007 21.3 -> 20.6, 600011 35.8 -> 37.6
+//   fp32, K 16:  n = 50000 5.3 -> 4.0, 100003 5.3 -> 4.1;  fp64 50000 4.6 ->
+//                3.9, 100003 4.9 -> 4.9;  K 12: fp32 50000 4.6 -> 4.0
+// so the split ends where the last of the four types stops gaining: 400000
+// rows, and 100000 rows for K <= 16.
+inline int split_waves(int32_t rows, int K)
+{
+    if (rows <= 100000 && K >= 10 && K <= kShortMax) return K < 13 ? 2 : 4;
+    if (rows <= 400000 && K > kShortMax) return K < 20 ? 2 : (K < 40 ? 4 : 8);
+    return 1;
+}
+
 template <typename TV, typename TX>
 using SpmvKernel = void (*)(int32_t, int32_t, int64_t, int32_t, const int32_t*, const TV*,
                             const TX*, TX*, int32_t, int32_t, DotArgs);
@@ -440,6 +571,17 @@ int spmv_run(int32_t rows, int32_t cols, int32_t num_diags, const int32_t* offs,
         return fail(DIAGPU_ERR_ARG, "%s: the dot epilogue needs x_size >= rows and its buffers",
                     name);
     if (lim == 0) K = 0;   // no column in range: y = 0 without touching values or x
+    const int S = dot || lim < Shape<TV, TX>::R ? 1 : split_waves(rows, K);
+    if (S > 1) {
+        const int32_t st = (int32_t)ceil_div<int64_t>(rows, 64 * Shape<TV, TX>::R);
+        const int32_t sx = ceil_div<int32_t>(st, kNumXcd);
+        hipLaunchKernelGGL((S == 2   ? spmv_split_kernel<TV, TX, 2>
+                            : S == 4 ? spmv_split_kernel<TV, TX, 4>
+                                     : spmv_split_kernel<TV, TX, 8>),
+                           dim3(sx * kNumXcd), dim3(64 * S), 0, as_stream(stream), rows, cols, lim,
+                           K, offs, vals, x, y, st, sx);
+        return check_launch(name);
+    }
     const int32_t tiles = spmv_tiles<TV, TX>(rows);
     const int32_t per_xcd = ceil_div<int32_t>(tiles, kNumXcd);
     const DotArgs da = dot ? *dot : DotArgs{nullptr, nullptr};

@@ -104,6 +104,35 @@ def test_poisson_closed_form_full_size(dev, dtype):
     assert torch.equal(y, missing)
 
 
+# The kernel whose waves share a tile and split its diagonals: K on both sides
+# of each number of waves (10, 13, 17, 20, 40), of the chunks of 8 per wave
+# (64, 65, 129) and of its row limits (100000 for K <= 16, 400000), rows on
+# the edges of the 64-lane tiles (256 rows in fp32, 128 in fp64), offsets in
+# random order that leave the matrix on both sides, and an x shorter than the
+# rows reach.  No element outside [0, min(cols, len(x))) may be used: x and
+# the matrix are NaN there.  Any order of K <= 166 fp32 terms stays within the
+# module's bound.
+@pytest.mark.parametrize("rows,K", [(1, 10), (63, 12), (255, 13), (256, 16), (257, 17),
+                                    (1000, 19), (1025, 20), (5000, 39), (5000, 40), (8191, 64),
+                                    (8193, 65), (20000, 129), (100000, 16), (100001, 16),
+                                    (100003, 64), (400000, 17), (400001, 17)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_split_diagonals(dev, oracle, rows, K, dtype):
+    rng = np.random.default_rng(rows + K)
+    npt = np.float32 if dtype == torch.float32 else np.float64
+    cols, xs = rows + 7, max(4, rows - rows // 5)
+    reach = max(K, min(rows + 9, 700))
+    off = rng.choice(np.arange(-reach, reach + 1), size=K, replace=False).astype(np.int32)
+    val = rng.uniform(-1, 1, (K, cols)).astype(npt)
+    x = rng.standard_normal(xs).astype(npt)
+    y64, absum = oracle.spmv_recon_ref64(rows, min(cols, xs), off,
+                                         np.ascontiguousarray(val[:, :xs]).reshape(-1), x)
+    val[:, xs:] = np.nan
+    y = gpu_spmv(dev, off, val.reshape(-1), rows, cols, x)
+    check_bound(y, y64, absum, TOL32 if dtype == torch.float32 else TOL64)
+    assert np.array_equal(y, gpu_spmv(dev, off, val.reshape(-1), rows, cols, x))
+
+
 def _random_rect(oracle, rng, rows, cols, offsets):
     H = np.zeros((rows, cols), np.float32)
     for d in offsets:
