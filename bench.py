@@ -379,6 +379,8 @@ def cpu_spgemm_baseline(plan, A, B, seconds: float, C_gpu=None):
 
 def kernel_legs(plan, complex_values: bool = False) -> list[str]:
     """Every numeric kernel that takes this plan."""
+    import torch
+
     from diagpu_amd import _lib
     names = ["gather"]
     if not complex_values and plan.band_info()[1].eligible:
@@ -391,6 +393,8 @@ def kernel_legs(plan, complex_values: bool = False) -> list[str]:
             names.append("astat")
         except _lib.DiagpuError:
             pass
+    if plan.uses_full(torch.complex64 if complex_values else torch.float32):
+        names.append("full")
     return names
 
 
@@ -568,7 +572,7 @@ def time_spgemm(cfg: int, seed: int, reps: int, complex_values: bool = False,
     flops = plan.info.useful_flops * (4 if complex_values else 1)   # complex MAC = 4 real
     auto, kernels = compare_kernels(plan, sets, reps, alg, flops, complex_values, rounds)
     ms = auto["numeric_ms"]
-    kern = plan.kernel_for(torch.complex64 if complex_values else torch.float32)
+    kern = plan.prepare(torch.complex64 if complex_values else torch.float32)
     rec = {
         "workload": name or (f"spgemm_cfg{cfg}" if cfg >= 4 else f"spgemm_HxH_cfg{cfg}"),
         "dtype": "c64" if complex_values else "f32", "n": A.n,
@@ -791,7 +795,7 @@ def time_gemm_diag(n: int = 4096, hb: int = 10, reps: int = 100, cpu_seconds: fl
         sets += [(DA.clone(), DB.clone(), torch.empty_like(C)) for _ in range(nsets - 1)]
     auto, kernels = compare_kernels(plan, sets, reps, alg, flops)
     ms = auto["numeric_ms"]
-    kern = plan.kernel_for()
+    kern = plan.prepare()
     rec = {"workload": f"gemm_diag_n{n}_hb{hb}", "n": n, "A_diags": len(offs),
            "B_diags": len(offs), "C_diags": plan.info.c_ndiag, "numeric_ms": round(ms, 5),
            "numeric_min_ms": auto["min_ms"], "numeric_max_ms": auto["max_ms"],

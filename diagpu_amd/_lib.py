@@ -72,6 +72,11 @@ class SpgemmInfo(C.Structure):
                 ("b_extent", C.c_int64)]
 
 
+class SpgemmShape(C.Structure):
+    _fields_ = [("a_off_min", C.c_int32), ("a_off_max", C.c_int32), ("b_off_min", C.c_int32),
+                ("b_off_max", C.c_int32), ("contiguous", C.c_int32)]
+
+
 _vp, _i32, _i64, _sz = C.c_void_p, C.c_int32, C.c_int64, C.c_size_t
 
 # name -> (restype, argtypes); every entry point declared in include/diagpu.h.
@@ -108,6 +113,22 @@ PROTOTYPES: dict[str, tuple] = {
         _vp, _sz,
         _vp, C.POINTER(_i32),
         C.POINTER(SpgemmInfo), _vp]),
+    "diagpu_spgemm_symbolic_shape": (C.c_int, [
+        _i32,
+        _vp, _vp, _vp, _i32,
+        _vp, _vp, _vp, _i32,
+        _vp, _vp, _vp, _i64,
+        _vp, _vp, _i64,
+        _vp,
+        _vp, _sz,
+        _vp, C.POINTER(_i32), C.POINTER(SpgemmShape),
+        C.POINTER(SpgemmInfo), _vp]),
+    "diagpu_spgemm_full_choice": (C.c_int, [_i32, _i32, _i32, _i64, _i64, C.POINTER(SpgemmShape),
+                                            _i32]),
+    "diagpu_spgemm_numeric_full_f32": (C.c_int, [_i32, _i32, _i32, _vp, _vp, _i32, _i32, _vp, _vp,
+                                                 _vp, _i64, _vp, _vp]),
+    "diagpu_spgemm_numeric_full_c64": (C.c_int, [_i32, _i32, _i32, _vp, _vp, _i32, _i32, _vp, _vp,
+                                                 _vp, _i64, _vp, _vp]),
     "diagpu_spgemm_symbolic_noalloc": (C.c_int, [
         _i32,
         _vp, _vp, _vp, _i32,

@@ -67,6 +67,7 @@ enum : int32_t {
     kFlagCCapacity = 16,
     kFlagPairCapacity = 32,
     kFlagFallback = 64,   // the one-launch path cannot hold the operands in LDS
+    kNotContiguous = 128, // no error: an operand's offsets are not lo, lo + 1, .. in order
 };
 
 struct SymState {
@@ -79,8 +80,11 @@ struct SymState {
     int32_t pad;
     int64_t a_extent;     // values A's starts and lengths address: max(start + length)
     int64_t b_extent;
+    int32_t a_min, a_max, b_min, b_max;   // offset ranges and contiguity: the
+    int32_t contiguous;                   // one-launch path only
+    int32_t spare;
 };
-static_assert(sizeof(SymState) == 64, "state is one 64-byte record");
+static_assert(sizeof(SymState) == 88, "state is one 88-byte record");
 
 struct Layout {
     int64_t nlk = 0;       // 2n - 1 offsets
@@ -142,6 +146,9 @@ __global__ __launch_bounds__(kBlock) void k_init(int32_t* __restrict__ alk, int6
         st->pad = 0;
         st->a_extent = 0;
         st->b_extent = 0;
+        st->a_min = st->a_max = st->b_min = st->b_max = 0;
+        st->contiguous = 0;
+        st->spare = 0;
     }
 }
 
@@ -572,7 +579,8 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
     bmax = combine_waves(s32[4], i32max);
     aext = combine_waves(s64[0], i64max);
     bext = combine_waves(s64[1], i64max);
-    auto report = [&](int32_t flags, int64_t nc, int64_t nnz, int64_t np, int64_t fl) {
+    auto report = [&](int32_t flags, int64_t nc, int64_t nnz, int64_t np, int64_t fl,
+                      int32_t contiguous = 0) {
         if (wg == 0 && tid == 0) {
             st->c_ndiag = nc;
             st->c_nnz = nnz;
@@ -583,6 +591,12 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
             st->pad = 0;
             st->a_extent = aext;
             st->b_extent = bext;
+            st->a_min = amin;
+            st->a_max = amax;
+            st->b_min = bmin;
+            st->b_max = bmax;
+            st->contiguous = contiguous;
+            st->spare = 0;
         }
     };
     if (bad) {
@@ -617,15 +631,18 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
     int32_t* cpfx = reinterpret_cast<int32_t*>(cbits + wc);
     int32_t* rows = cpfx + wc;                       // the slice's C offsets
 
-    // a bit already set is a repeated offset
-    int32_t dup = 0;
+    // a bit already set is a repeated offset; distinct offsets lo + index are
+    // a contiguous band in order
+    int32_t dup = na && nb ? 0 : kNotContiguous;
     for (int a = tid; a < na; a += kFastBlock) {
         const int64_t q = (int64_t)aoff[a] - amin;
+        dup |= q == a ? 0 : kNotContiguous;
         const uint32_t m = 1u << (q & 31);
         if (atomicOr(&abits[q >> 5], m) & m) dup |= kFlagADup;
     }
     for (int b = tid; b < nb; b += kFastBlock) {
         const int64_t q = (int64_t)boff[b] - bmin;
+        dup |= q == b ? 0 : kNotContiguous;
         const uint32_t m = 1u << (q & 31);
         if (atomicOr(&bbits[q >> 5], m) & m) dup |= kFlagBDup;
     }
@@ -677,6 +694,8 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
     dup = combine_waves(s32[5], i32or);
     np = combine_waves(s64[2], i64add);
     fl = combine_waves(s64[3], i64add);
+    const int32_t contiguous = (dup & kNotContiguous) ? 0 : 1;
+    dup &= ~kNotContiguous;
     if (dup) {
         report(dup, 0, 0, 0, 0);
         return;
@@ -768,7 +787,7 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
     int32_t flags = 0;
     if (nC > c_cap) flags |= kFlagCCapacity;
     if (np > p_cap) flags |= kFlagPairCapacity;
-    report(flags, nC, nnz, np, fl);
+    report(flags, nC, nnz, np, fl, contiguous);
     if (flags) return;
     if (records && wg == 0 && tid == 0)   // the 4 ints after the records
         reinterpret_cast<int4*>(records)[np] = int4{0, 0, amin, amax};
@@ -961,7 +980,7 @@ int fast_lds_allowed(const char* fn)
     return DIAGPU_OK;
 }
 
-// The two entry points below share this runner.  workspace == nullptr asks
+// The entry points below share this runner.  workspace == nullptr asks
 // for the file-scope scratch array (diagpu_spgemm_symbolic_noalloc).
 int run_symbolic(
     const char* fn, int32_t n,
@@ -971,7 +990,7 @@ int run_symbolic(
     int64_t* pair_ptr, diagpu_gpair* pairs, int64_t pair_capacity,
     int32_t* c_lookup, bool use_scratch,
     void* workspace, size_t workspace_bytes,
-    int32_t* records, int32_t* records_status,
+    int32_t* records, int32_t* records_status, diagpu_spgemm_shape* shape,
     diagpu_spgemm_info* info, void* stream)
 {
     if (!info) return fail(DIAGPU_ERR_ARG, "%s: info is NULL", fn);
@@ -1119,6 +1138,7 @@ int run_symbolic(
     info->useful_flops = h.useful_flops;
     info->a_extent = h.a_extent;
     info->b_extent = h.b_extent;
+    if (shape) *shape = diagpu_spgemm_shape{h.a_min, h.a_max, h.b_min, h.b_max, h.contiguous};
     if (h.flags & (kFlagAOffset | kFlagBOffset))
         return fail(DIAGPU_ERR_OFFSET, "%s: an %s offset has |d| >= n=%d or length != n - |d|",
                     fn, (h.flags & kFlagAOffset) ? "A" : "B", n);
@@ -1172,7 +1192,8 @@ DIAGPU_API int diagpu_spgemm_symbolic(
     return diagpu::run_symbolic("diagpu_spgemm_symbolic", n, A_off, A_len, A_starts, a_ndiag,
                                 B_off, B_len, B_starts, b_ndiag, C_off, C_len, C_starts,
                                 c_capacity, pair_ptr, pairs, pair_capacity, c_lookup, false,
-                                workspace, workspace_bytes, nullptr, nullptr, info, stream);
+                                workspace, workspace_bytes, nullptr, nullptr, nullptr, info,
+                                stream);
 }
 
 DIAGPU_API int diagpu_spgemm_symbolic_astat(
@@ -1191,7 +1212,29 @@ DIAGPU_API int diagpu_spgemm_symbolic_astat(
     return diagpu::run_symbolic("diagpu_spgemm_symbolic_astat", n, A_off, A_len, A_starts,
                                 a_ndiag, B_off, B_len, B_starts, b_ndiag, C_off, C_len, C_starts,
                                 c_capacity, pair_ptr, pairs, pair_capacity, c_lookup, false,
-                                workspace, workspace_bytes, records, records_status, info, stream);
+                                workspace, workspace_bytes, records, records_status, nullptr, info,
+                                stream);
+}
+
+DIAGPU_API int diagpu_spgemm_symbolic_shape(
+    int32_t n,
+    const int32_t* A_off, const int32_t* A_len, const int64_t* A_starts, int32_t a_ndiag,
+    const int32_t* B_off, const int32_t* B_len, const int64_t* B_starts, int32_t b_ndiag,
+    int32_t* C_off, int32_t* C_len, int64_t* C_starts, int64_t c_capacity,
+    int64_t* pair_ptr, diagpu_gpair* pairs, int64_t pair_capacity,
+    int32_t* c_lookup,
+    void* workspace, size_t workspace_bytes,
+    int32_t* records, int32_t* records_status,
+    diagpu_spgemm_shape* shape,
+    diagpu_spgemm_info* info, void* stream)
+{
+    if (!shape)
+        return diagpu::fail(DIAGPU_ERR_ARG, "diagpu_spgemm_symbolic_shape: shape is NULL");
+    return diagpu::run_symbolic("diagpu_spgemm_symbolic_shape", n, A_off, A_len, A_starts,
+                                a_ndiag, B_off, B_len, B_starts, b_ndiag, C_off, C_len, C_starts,
+                                c_capacity, pair_ptr, pairs, pair_capacity, c_lookup, false,
+                                workspace, workspace_bytes, records, records_status, shape, info,
+                                stream);
 }
 
 DIAGPU_API int diagpu_spgemm_symbolic_noalloc(
@@ -1205,7 +1248,7 @@ DIAGPU_API int diagpu_spgemm_symbolic_noalloc(
     return diagpu::run_symbolic("diagpu_spgemm_symbolic_noalloc", n, A_off, A_len, A_starts,
                                 a_ndiag, B_off, B_len, B_starts, b_ndiag, C_off, C_len, C_starts,
                                 c_capacity, pair_ptr, pairs, pair_capacity, c_lookup, true,
-                                nullptr, 0, nullptr, nullptr, info, stream);
+                                nullptr, 0, nullptr, nullptr, nullptr, info, stream);
 }
 
 }  // extern "C"

@@ -60,8 +60,7 @@ class SpgemmPlan:
         if want_lookup:
             parts.append(("lookup", torch.int32, 2 * self.n - 1))
         # where the A-stationary kernel may take the plan, the symbolic call
-        # also builds that kernel's records (diagpu_spgemm_symbolic_astat):
-        # one stream sync for both
+        # also builds that kernel's records: one stream sync for both
         self._fused = (4096 <= self.n < 1 << 30 and self.p_cap < 1 << 28
                        and na <= max(_lib.ASTAT_MAX_A, _lib.ASTAT_MAX_A_C64))
         if self._fused:
@@ -80,8 +79,9 @@ class SpgemmPlan:
         self._band = None
         self._astat = None
         self._rstat = C.c_int32(0)
-        self._sym_fn = getattr(_lib.load(), "diagpu_spgemm_symbolic_astat" if self._fused
-                               else "diagpu_spgemm_symbolic")
+        self.shape = _lib.SpgemmShape()
+        self._full = {}
+        self._sym_fn = _lib.load().diagpu_spgemm_symbolic_shape
         self._sym_args, self._sym_caps, self._sym_ops = None, None, ()
         self.symbolic()
 
@@ -107,11 +107,12 @@ class SpgemmPlan:
 
     def symbolic(self) -> None:
         """(Re)builds the C structure and pair plan from the operands'
-        offsets, lengths and starts (diagpu_spgemm_symbolic, or
-        diagpu_spgemm_symbolic_astat with the A-stationary records; one
-        stream sync)."""
+        offsets, lengths and starts (diagpu_spgemm_symbolic_shape, with the
+        A-stationary records where that kernel may take the plan; one stream
+        sync)."""
         self._band = None
         self._astat = None
+        self._full = {}
         A, B = self.A, self.B
         ops = (A.offsets, A.lengths, A.starts, B.offsets, B.lengths, B.starts)
         if (self._sym_caps != (self.c_cap, self.p_cap)
@@ -130,9 +131,8 @@ class SpgemmPlan:
                               self.c_cap, self._addr("ptr"), self._addr("pairs"), self.p_cap,
                               self._addr("lookup"), self._addr("workspace"),
                               self._parts["workspace"][2])
-            if self._fused:
-                self._sym_args += (self._addr("records"), C.byref(self._rstat))
-            self._sym_args += (C.byref(self.info),)
+            self._sym_args += (self._addr("records"), C.byref(self._rstat), C.byref(self.shape),
+                               C.byref(self.info))
             self._sym_caps = (self.c_cap, self.p_cap)
         st = self._sym_fn(*self._sym_args, _stream_handle(self.stream))
         if st:
@@ -167,8 +167,9 @@ class SpgemmPlan:
     def prepare(self, dtype=torch.float32) -> str:
         """Runs now, on the plan's stream, the per-plan set-up of the kernel
         `numeric` takes by default for `dtype` (band or A-stationary
-        prepare, each one stream sync), and returns that kernel's name."""
-        return self.kernel_for(dtype)
+        prepare, each one stream sync; none for "full"), and returns that
+        kernel's name."""
+        return "full" if self.uses_full(dtype) else self.kernel_for(dtype)
 
     def hand_over(self, stream) -> None:
         """Continue the plan on `stream` (a torch stream): its buffers are
@@ -324,8 +325,24 @@ class SpgemmPlan:
         issued = 2 * 16 * 16 * 4 * info.mfma_blocks * 4 * -(-self.n // 64)
         return self.info.useful_flops / issued
 
+    def uses_full(self, dtype=torch.float32) -> bool:
+        """Whether "auto" runs the contiguous-band kernel
+        (diagpu_spgemm_full_choice: both operands hold every offset of a range
+        in ascending order, they fit in LDS, and each C diagonal takes enough
+        entries): it then stands in for the kernel that kernel_for names."""
+        v = self._full.get(dtype)
+        if v is None:
+            inf = self.info
+            v = dtype in (torch.float32, torch.complex64) and bool(
+                _lib.load().diagpu_spgemm_full_choice(
+                    self.n, self.A.offsets.numel(), self.B.offsets.numel(), inf.c_ndiag,
+                    inf.n_pairs, C.byref(self.shape), int(dtype == torch.complex64)))
+            self._full[dtype] = v
+        return v
+
     def kernel_for(self, dtype=torch.float32) -> str:
-        """The kernel "auto" runs: "band", "astat" or "gather"."""
+        """The general kernel "auto" runs: "band", "astat" or "gather" (where
+        uses_full holds, the contiguous-band kernel runs in its place)."""
         if self.uses_band(dtype):
             return "band"
         if self.uses_astat(dtype):
@@ -335,10 +352,11 @@ class SpgemmPlan:
     def numeric(self, A_vals: torch.Tensor, B_vals: torch.Tensor, C_vals: torch.Tensor,
                 kernel: str = "auto") -> None:
         """C values for the plan's structure; float32 or complex64 (all three
-        tensors the same dtype).  kernel: "auto" (kernel_for), "gather" (any
-        plan), "band" (fp32, narrow bands) or "astat" (at most
-        DIAGPU_ASTAT_MAX_A A diagonals, DIAGPU_ASTAT_MAX_A_C64 for complex
-        values), which all return the same bits, or
+        tensors the same dtype).  kernel: "auto" ("full" where uses_full,
+        else kernel_for), "gather" (any plan), "band" (fp32, narrow bands),
+        "astat" (at most DIAGPU_ASTAT_MAX_A A diagonals,
+        DIAGPU_ASTAT_MAX_A_C64 for complex values) or "full" (contiguous
+        bands in ascending order), which all return the same bits, or
         "band_mfma" (fp32, narrow bands on the matrix cores: the same values
         to rounding, finite operands)."""
         dt = A_vals.dtype
@@ -346,7 +364,7 @@ class SpgemmPlan:
                 torch.complex64: "diagpu_spgemm_numeric_c64"}.get(dt)
         if name is None:
             raise TypeError(f"unsupported value dtype {dt}")
-        if kernel not in ("auto", "gather", "band", "astat", "band_mfma"):
+        if kernel not in ("auto", "gather", "band", "astat", "full", "band_mfma"):
             raise ValueError(f"unknown kernel {kernel!r}")
         _check_dev(A_vals, dt, "A_vals")
         _check_dev(B_vals, dt, "B_vals")
@@ -358,7 +376,18 @@ class SpgemmPlan:
         if C_vals.numel() < self.info.c_nnz:
             raise ValueError(f"C_vals has {C_vals.numel()} elements, needs {self.info.c_nnz}")
         if kernel == "auto":
-            kernel = self.kernel_for(dt)
+            kernel = "full" if self.uses_full(dt) else self.kernel_for(dt)
+        if kernel == "full":
+            if not self.shape.contiguous:
+                raise ValueError("the full kernel takes contiguous bands in ascending order")
+            A, B = self.A, self.B
+            _lib.call("diagpu_spgemm_numeric_full_f32" if dt == torch.float32
+                      else "diagpu_spgemm_numeric_full_c64", self.n, self.shape.a_off_min,
+                      A.offsets.numel(), A.starts.data_ptr(), A_vals.data_ptr(),
+                      self.shape.b_off_min, B.offsets.numel(), B.starts.data_ptr(),
+                      B_vals.data_ptr(), self._addr("C_starts"), self.info.c_ndiag,
+                      C_vals.data_ptr(), _stream_handle(self.stream))
+            return
         if kernel in ("band", "band_mfma") and dt != torch.float32:
             raise TypeError(f"the {kernel} kernel is fp32")
         if kernel == "band_mfma":

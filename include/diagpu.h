@@ -406,6 +406,56 @@ DIAGPU_API int diagpu_spgemm_symbolic_astat(
     int32_t* records, int32_t* records_status,
     diagpu_spgemm_info* info, void* stream);
 
+/* What the symbolic phase saw of the operands' offsets (host memory). */
+typedef struct diagpu_spgemm_shape {
+    int32_t a_off_min, a_off_max;   /* smallest and largest A offset            */
+    int32_t b_off_min, b_off_max;   /* smallest and largest B offset            */
+    int32_t contiguous;             /* 1: A holds every offset a_off_min ..     */
+                                    /* a_off_max and B every offset b_off_min   */
+                                    /* .. b_off_max, each in ascending order;   */
+                                    /* 0: otherwise, or not looked at (operands */
+                                    /* beyond the one-launch path, or empty)    */
+} diagpu_spgemm_shape;
+
+/* diagpu_spgemm_symbolic_astat with the operands' shape (host out) in the
+ * same read-back.  records may be NULL (records_status is then not written
+ * and may be NULL too): the plan alone, as diagpu_spgemm_symbolic.  No
+ * reference counterpart. */
+DIAGPU_API int diagpu_spgemm_symbolic_shape(
+    int32_t n,
+    const int32_t* A_off, const int32_t* A_len, const int64_t* A_starts, int32_t a_ndiag,
+    const int32_t* B_off, const int32_t* B_len, const int64_t* B_starts, int32_t b_ndiag,
+    int32_t* C_off, int32_t* C_len, int64_t* C_starts, int64_t c_capacity,
+    int64_t* pair_ptr, diagpu_gpair* pairs, int64_t pair_capacity,
+    int32_t* c_lookup,
+    void* workspace, size_t workspace_bytes,
+    int32_t* records, int32_t* records_status,
+    diagpu_spgemm_shape* shape,
+    diagpu_spgemm_info* info, void* stream);
+
+/* The numeric phase of diagpu_spgemm_numeric_f32 / _c64 (same C, bit for bit)
+ * for contiguous bands in ascending order (shape->contiguous), as
+ * make_banded and gemm_diag have them: register tiles of C over operands
+ * staged in LDS, no plan entries read.  nA + nB - 1 = c_ndiag C diagonals,
+ * all sums of offsets inside (-n, n) (else DIAGPU_ERR_ARG); operands that do
+ * not fit in LDS are refused with DIAGPU_ERR_CAPACITY (nA at most 69). */
+DIAGPU_API int diagpu_spgemm_numeric_full_f32(
+    int32_t n, int32_t a_off_min, int32_t nA, const int64_t* A_starts, const float* A_vals,
+    int32_t b_off_min, int32_t nB, const int64_t* B_starts, const float* B_vals,
+    const int64_t* C_starts, int64_t c_ndiag, float* C_vals, void* stream);
+DIAGPU_API int diagpu_spgemm_numeric_full_c64(
+    int32_t n, int32_t a_off_min, int32_t nA, const int64_t* A_starts,
+    const diagpu_complex64* A_vals, int32_t b_off_min, int32_t nB, const int64_t* B_starts,
+    const diagpu_complex64* B_vals, const int64_t* C_starts, int64_t c_ndiag,
+    diagpu_complex64* C_vals, void* stream);
+
+/* 1 where the contiguous-band kernel takes a plan and is the faster one (the
+ * automatic choice of the Python and C++ plans), else 0.  Host only: no
+ * status, no HIP call. */
+DIAGPU_API int diagpu_spgemm_full_choice(int32_t n, int32_t nA, int32_t nB, int64_t c_ndiag,
+                                         int64_t n_pairs, const diagpu_spgemm_shape* shape,
+                                         int32_t complex_values);
+
 /* The numeric phase of diagpu_spgemm_numeric_f32 (same C, bit for bit) with
  * each workgroup holding one block of 64 R rows of every A diagonal (plus the
  * 32 rows before it; R = 4, 8 or 16 rows per lane, chosen per launch) in LDS

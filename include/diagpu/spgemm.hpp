@@ -245,7 +245,8 @@ inline FlatPlan build_flat_plan(int n, const std::vector<int>& A_off, const std:
 namespace diagpu {
 
 // Which numeric kernel SpgemmPlan::numeric runs for fp32 values.
-//   Auto:        Band where the plan qualifies (SpgemmPlan::uses_band), else
+//   Auto:        Full where the plan qualifies (SpgemmPlan::uses_full), else
+//                Band where it does (uses_band), else
 //                AStationary where it qualifies (uses_astat), else Gather;
 //   Gather:      diagpu_spgemm_numeric_f32, any plan;
 //   Band:        diagpu_spgemm_numeric_band_f32 (operands staged in LDS;
@@ -253,7 +254,7 @@ namespace diagpu {
 //   AStationary: diagpu_spgemm_numeric_astat_f32 (A held in LDS; at most
 //                DIAGPU_ASTAT_MAX_A A diagonals, else DIAGPU_ERR_CAPACITY).
 // All return the same bits.
-enum class NumericKernel { Auto, Gather, Band, AStationary };
+enum class NumericKernel { Auto, Gather, Band, AStationary, Full };
 
 // Device-resident C = A * B for HM operands whose offsets, lengths and starts
 // are device arrays: the plan is built once (symbolic), numeric() may run
@@ -279,28 +280,23 @@ public:
         check(diagpu_spgemm_symbolic_workspace(n, a_ndiag, b_ndiag, &ws_bytes));
         DeviceArray<char> ws(ws_bytes);
         // Where the A-stationary kernel may take the plan, the symbolic call
-        // also builds its records (diagpu_spgemm_symbolic_astat: one stream
-        // synchronisation for both).
+        // also builds its records (one stream synchronisation for both).
         const bool fused = int64_t(n) >= 4096 && int64_t(n) < (int64_t(1) << 30) &&
                            pcap < (int64_t(1) << 28) &&
                            a_ndiag <= std::max(DIAGPU_ASTAT_MAX_A, DIAGPU_ASTAT_MAX_A_C64);
         int32_t rstat = DIAGPU_OK;
+        if (fused) records_.resize(size_t(4 * pcap + 4));
+        check(diagpu_spgemm_symbolic_shape(
+            n, dA_off, dA_len, dA_starts, a_ndiag, dB_off, dB_len, dB_starts, b_ndiag,
+            C_off_.data(), C_len_.data(), C_starts_.data(), ccap, ptr_.data(), pairs_.data(),
+            pcap, want_lookup ? lookup_.data() : nullptr, ws.data(), ws_bytes,
+            fused ? records_.data() : nullptr, &rstat, &shape_, &info_, stream));
         if (fused) {
-            records_.resize(size_t(4 * pcap + 4));
-            check(diagpu_spgemm_symbolic_astat(
-                n, dA_off, dA_len, dA_starts, a_ndiag, dB_off, dB_len, dB_starts, b_ndiag,
-                C_off_.data(), C_len_.data(), C_starts_.data(), ccap, ptr_.data(), pairs_.data(),
-                pcap, want_lookup ? lookup_.data() : nullptr, ws.data(), ws_bytes,
-                records_.data(), &rstat, &info_, stream));
             if (rstat != DIAGPU_OK && rstat != DIAGPU_ERR_CAPACITY) check(rstat);
             astat_prepared_ = rstat == DIAGPU_OK;
-        } else {
-            check(diagpu_spgemm_symbolic(n, dA_off, dA_len, dA_starts, a_ndiag, dB_off, dB_len,
-                                         dB_starts, b_ndiag, C_off_.data(), C_len_.data(),
-                                         C_starts_.data(), ccap, ptr_.data(), pairs_.data(), pcap,
-                                         want_lookup ? lookup_.data() : nullptr, ws.data(),
-                                         ws_bytes, &info_, stream));
         }
+        full_auto_ = full_choice(a_ndiag, b_ndiag, 0);
+        full_auto_c64_ = full_choice(a_ndiag, b_ndiag, 1);
         nA_ = a_ndiag;
         nB_ = b_ndiag;
         A_off_.resize(a_ndiag);
@@ -359,6 +355,11 @@ public:
     // diagonals, 4096 <= n < 2^30, and n >= 2^16 or >= 3 entries per A diagonal.
     bool uses_astat_c64() const { return astat_auto_c64_; }
 
+    // True where NumericKernel::Auto runs the contiguous-band kernel in the
+    // place of the ones above (diagpu_spgemm_full_choice).
+    bool uses_full() const { return full_auto_; }
+    bool uses_full_c64() const { return full_auto_c64_; }
+
     // C_vals (device, info().c_nnz values) = A * B; asynchronous on `stream`
     // (NumericKernel::Band or AStationary on a plan not yet prepared for it
     // synchronises once to prepare).
@@ -366,8 +367,17 @@ public:
                  NumericKernel kernel = NumericKernel::Auto) const
     {
         if (kernel == NumericKernel::Auto)
-            kernel = uses_band() ? NumericKernel::Band
-                                 : (uses_astat() ? NumericKernel::AStationary : NumericKernel::Gather);
+            kernel = uses_full() ? NumericKernel::Full
+                     : uses_band()
+                         ? NumericKernel::Band
+                         : (uses_astat() ? NumericKernel::AStationary : NumericKernel::Gather);
+        if (kernel == NumericKernel::Full) {
+            require_contiguous();
+            check(diagpu_spgemm_numeric_full_f32(n_, shape_.a_off_min, nA_, A_starts_.data(), dA_vals,
+                                                 shape_.b_off_min, nB_, B_starts_.data(), dB_vals,
+                                                 C_starts_.data(), info_.c_ndiag, dC_vals, stream));
+            return;
+        }
         if (kernel == NumericKernel::AStationary) {
             if (!astat_prepared_) prepare_astat(stream);
             check(diagpu_spgemm_numeric_astat_f32(
@@ -390,14 +400,24 @@ public:
     }
 
     // The same product with complex64 operands and C (same plan): Auto runs
-    // the A-stationary kernel where uses_astat_c64(), else the gather; Band
+    // the contiguous-band kernel where uses_full_c64(), else the A-stationary
+    // kernel where uses_astat_c64(), else the gather; Band
     // is refused (fp32 only) with DIAGPU_ERR_ARG.
     void numeric(const diagpu_complex64* dA_vals, const diagpu_complex64* dB_vals,
                  diagpu_complex64* dC_vals, hipStream_t stream = 0,
                  NumericKernel kernel = NumericKernel::Auto) const
     {
         if (kernel == NumericKernel::Auto)
-            kernel = uses_astat_c64() ? NumericKernel::AStationary : NumericKernel::Gather;
+            kernel = uses_full_c64() ? NumericKernel::Full
+                     : uses_astat_c64() ? NumericKernel::AStationary
+                                        : NumericKernel::Gather;
+        if (kernel == NumericKernel::Full) {
+            require_contiguous();
+            check(diagpu_spgemm_numeric_full_c64(n_, shape_.a_off_min, nA_, A_starts_.data(), dA_vals,
+                                                 shape_.b_off_min, nB_, B_starts_.data(), dB_vals,
+                                                 C_starts_.data(), info_.c_ndiag, dC_vals, stream));
+            return;
+        }
         if (kernel == NumericKernel::Band)
             throw Error(DIAGPU_ERR_ARG, "SpgemmPlan::numeric: the band kernel takes fp32 values only");
         if (kernel == NumericKernel::AStationary) {
@@ -467,6 +487,17 @@ private:
             check_hip(hipMemcpyAsync(dst, src, size_t(count) * sizeof(T), hipMemcpyDeviceToDevice, stream),
                       "hipMemcpyAsync");
     }
+    bool full_choice(int a_ndiag, int b_ndiag, int complex_values) const
+    {
+        return diagpu_spgemm_full_choice(n_, a_ndiag, b_ndiag, info_.c_ndiag, info_.n_pairs, &shape_,
+                                         complex_values) != 0;
+    }
+    void require_contiguous() const
+    {
+        if (!shape_.contiguous)
+            throw Error(DIAGPU_ERR_ARG, "SpgemmPlan::numeric: the operands are no contiguous bands in "
+                                        "ascending order");
+    }
     void prepare_band(hipStream_t stream) const
     {
         entries_.resize(size_t(4 * info_.n_pairs + 8));
@@ -491,6 +522,9 @@ private:
     DeviceArray<int64_t> C_starts_, ptr_, A_starts_, B_starts_;
     DeviceArray<diagpu_gpair> pairs_;
     diagpu_spgemm_info info_{};
+    diagpu_spgemm_shape shape_{};
+    bool full_auto_ = false;
+    bool full_auto_c64_ = false;
     bool band_auto_ = false;
     bool astat_auto_ = false;
     bool astat_auto_c64_ = false;

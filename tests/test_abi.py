@@ -283,3 +283,40 @@ def test_package_modules_import():
     assert {"spgemm", "chain", "spmv", "krylov", "workloads", "_lib", "build"} <= set(names)
     for name in names:
         importlib.import_module(f"diagpu_amd.{name}")
+
+
+def test_full_choice_is_host_logic():
+    """The contiguous-band rule: only whole contiguous products, only operands
+    that fit in LDS, from the stated number of entries per C diagonal."""
+    fn = _lib.load().diagpu_spgemm_full_choice
+
+    def take(n, a0, na, b0, nb, cplx=0, contiguous=1, nc=None, pairs=None):
+        sh = _lib.SpgemmShape(a0, a0 + na - 1, b0, b0 + nb - 1, contiguous)
+        return fn(n, na, nb, na + nb - 1 if nc is None else nc,
+                  na * nb if pairs is None else pairs, C.byref(sh), cplx)
+
+    assert take(100000, -16, 33, -16, 33) == 1
+    assert take(100000, -16, 33, -16, 33, contiguous=0) == 0
+    assert take(100000, -16, 33, -16, 33, nc=64) == 0
+    assert take(100000, -16, 33, -16, 33, pairs=1088) == 0
+    assert take(20, -10, 21, -10, 21) == 0            # sums reach beyond +-19
+    assert take(21, -10, 21, -10, 21) == 1
+    assert take(100000, -3, 7, -3, 7) == 0 and take(100000, -3, 7, -3, 7, cplx=1) == 1
+    assert take(5000, -2, 5, -2, 5) == 1 and take(5000, -1, 3, -1, 3) == 0
+    assert take(5000, -34, 69, -3, 7) == 1 and take(5000, -35, 70, -3, 7) == 0
+    assert take(5000, -3, 7, -2000, 4000) == 0        # beyond LDS
+    assert fn(100, 3, 3, 5, 9, None, 0) == 0
+
+
+def test_full_argument_errors():
+    f = C.c_void_p(0x1000)   # never dereferenced: validation fails first
+    name = "diagpu_spgemm_numeric_full_f32"
+    ok = (100, -1, 3, f, f, -1, 3, f, f, f, 5, f, None)
+    for at, bad in ((0, 0), (2, 0), (3, None), (4, None), (6, 0), (8, None), (9, None), (10, 4),
+                    (11, None), (1, -100), (5, 98)):
+        args = list(ok)
+        args[at] = bad
+        assert _status(name, *args) == _lib.ERR_ARG, at
+    assert _status(name, 10000, -100, 201, f, f, -1, 3, f, f, f, 203, f, None) == _lib.ERR_CAPACITY
+    assert _status("diagpu_spgemm_symbolic_shape", 4, f, f, f, 1, f, f, f, 1, f, f, f, 1, f, f, 1,
+                   None, f, 1 << 20, None, None, None, C.byref(_lib.SpgemmInfo()), None) == _lib.ERR_ARG

@@ -914,3 +914,80 @@ def test_band_mfma_refuses_wide_spans(dev):
     with pytest.raises(_lib.DiagpuError) as e:
         p4.numeric(A4.values, B4.values, Cv, kernel="band_mfma")
     assert e.value.status == _lib.ERR_CAPACITY
+
+
+# The contiguous-band kernel against the gather, bit for bit: rows on the edges
+# of its 64-, 128- and 256-row blocks and of its form limits (20000, 65536),
+# bands on both sides of its tiles of 4, 6 and 8 diagonals, wider than they
+# are high, off the main diagonal, and as wide as n; the largest A it takes.
+FULL_SHAPES = [
+    (1, 0, 1, 0, 1), (5, -2, 3, -2, 2), (63, -3, 4, -3, 4), (64, -5, 11, -4, 9),
+    (65, 0, 8, -7, 8), (255, -30, 61, 0, 9), (1000, -1, 2, -40, 81), (4097, -10, 21, -10, 21),
+    (9999, -34, 69, -3, 7), (20000, -16, 33, -16, 33), (20011, 7, 20, -25, 9),
+    (20161, -4, 8, -4, 9), (65536, -16, 33, -16, 33), (65537, -7, 15, -8, 17),
+    (65791, -8, 30, -20, 40), (100000, -3, 7, -24, 49),
+]
+
+
+@pytest.mark.parametrize("n,a0,na,b0,nb", FULL_SHAPES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.complex64])
+def test_full_same_bits_as_gather(dev, oracle, n, a0, na, b0, nb, dtype):
+    A = workloads.hm_random(n, range(a0, a0 + na), seed=n, device=dev)
+    B = workloads.hm_random(n, range(b0, b0 + nb), seed=n + 1, device=dev)
+    av, bv = A.values, B.values
+    if dtype == torch.complex64:
+        av = torch.complex(av, torch.roll(av, 3)).contiguous()
+        bv = torch.complex(bv, torch.roll(bv, 5)).contiguous()
+    plan = SpgemmPlan(A, B)
+    assert plan.shape.contiguous
+    assert (plan.shape.a_off_min, plan.shape.b_off_max) == (a0, b0 + nb - 1)
+    word = lambda v: torch.view_as_real(v).view(torch.int32) if v.is_complex() else v.view(torch.int32)
+
+    def run(x, y):
+        C = torch.full((plan.info.c_nnz,), float("nan"), dtype=dtype, device=dev)
+        plan.numeric(x, y, C, kernel="full")
+        return C
+
+    want = plan.multiply(av, bv, kernel="gather")
+    assert torch.equal(word(run(av, bv)), word(want))
+    auto = plan.multiply(av, bv)
+    assert torch.equal(word(auto), word(want))
+    # an infinity and a NaN in either operand reach the same C values and no
+    # other (the payload of a NaN is not compared)
+    rng = np.random.default_rng(n)
+    for which in (0, 1):
+        x, y = av.clone(), bv.clone()
+        v = (x, y)[which]
+        for bad in (float("inf"), float("nan")):
+            v[int(rng.integers(v.numel()))] = bad
+        got, ref = run(x, y), plan.multiply(x, y, kernel="gather")
+        if dtype == torch.complex64:
+            got, ref = torch.view_as_real(got), torch.view_as_real(ref)
+        assert torch.equal(torch.isnan(got), torch.isnan(ref))
+        assert torch.equal(torch.nan_to_num(got, nan=0.0), torch.nan_to_num(ref, nan=0.0))
+
+
+def test_full_only_for_contiguous_bands_in_order(dev):
+    """Holes, another order, or sums clipped at n: the general kernels."""
+    n = 70000
+    band = list(range(-10, 11))
+    assert SpgemmPlan(workloads.hm_random(n, band, 1, dev),
+                      workloads.hm_random(n, band, 2, dev)).uses_full()
+    H = workloads.hm_random(n, [d for d in band if d != 4], 1, dev)
+    B = workloads.hm_random(n, band, 2, dev)
+    for A in (H, workloads.HM(n, B.offsets.flip(0).contiguous(), B.lengths.flip(0).contiguous(),
+                              B.starts.flip(0).contiguous(), B.values)):
+        plan = SpgemmPlan(A, B)
+        assert not plan.shape.contiguous and not plan.uses_full()
+        with pytest.raises(ValueError):
+            plan.multiply(A.values, B.values, kernel="full")
+        assert torch.equal(plan.multiply(A.values, B.values),
+                           plan.multiply(A.values, B.values, kernel="gather"))
+    n = 30
+    A = workloads.hm_random(n, range(-20, 21), 3, dev)
+    plan = SpgemmPlan(A, A)
+    assert plan.shape.contiguous and not plan.uses_full()
+    with pytest.raises(_lib.DiagpuError):
+        plan.multiply(A.values, A.values, kernel="full")
+    assert torch.equal(plan.multiply(A.values, A.values),
+                       plan.multiply(A.values, A.values, kernel="gather"))
