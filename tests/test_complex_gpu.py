@@ -232,6 +232,122 @@ def test_propagator_pageable_readback(dev):
     assert torch.equal(out, pinned.psi)
 
 
+# The one-launch and the fused-step propagators against exp(-i t H) psi_0 by a
+# Taylor series in complex128: numbers of diagonals on both sides of each
+# kernel's (3, 5, 7, 9), rows on the edges of their workgroups (256, 512) and
+# of their ranges (16384, 131072, 262144, 500000), offsets that leave the
+# matrix altogether, m = 1 and 2.  |t| ||H|| <= 1, where m = 12 steps leave a
+# truncation below 1e-9; fp32 Lanczos vectors bound the rest: 12 steps of a few
+# units of 2^-24 each, well inside 2e-6.
+@pytest.mark.parametrize("n,pos", [
+    (5, [0, 1]), (256, [0, 255]), (257, [0, 1, 16]), (4097, [0, 1, 2, 64]), (16384, [1]),
+    (16385, [0, 1, 2, 3, 100]), (131072, [0, 5]), (131073, [0, 1, 300]),
+    (262144, [0, 1, 512, 513]), (262145, [0, 1, 512]), (262200, [0, 1, 512, 513]),
+    (300007, [0, 1, 2, 512, 700]), (500000, [0, 1]), (500001, [0, 707])])
+@pytest.mark.parametrize("complex_values", [True, False])
+def test_propagator_launch_forms(dev, n, pos, complex_values):
+    g = torch.Generator(device=dev).manual_seed(n)
+    dt = torch.complex64 if complex_values else torch.float32
+    offs, rows = [], []
+    scale = 1.0 / (2 * len(pos))
+    for d in pos:
+        v = (torch.rand(n, generator=g, device=dev) * 2 - 1) * scale       # H[r, r + d]
+        if complex_values and d:
+            v = v * torch.polar(torch.ones_like(v), torch.arange(n, device=dev) * 0.3)
+        v = v.to(dt)
+        if d == 0:
+            offs.append(0)
+            rows.append(v)
+            continue
+        up = torch.zeros(n, dtype=dt, device=dev)
+        dn = torch.zeros(n, dtype=dt, device=dev)
+        up[d:] = v[:n - d]              # column r + d of row r
+        dn[:n - d] = v[:n - d].conj()   # column r of row r + d
+        offs += [d, -d]
+        rows += [up, dn]
+    if len(offs) in (2, 4, 6, 8):       # a diagonal outside the matrix adds nothing
+        offs.append(n + 3)
+        rows.append(torch.full((n,), float("nan"), device=dev, dtype=dt))
+    o = torch.tensor(offs, dtype=torch.int32, device=dev)
+    v = torch.cat(rows)
+    psi0 = torch.complex(torch.randn(n, generator=g, device=dev),
+                         torch.randn(n, generator=g, device=dev))
+
+    def apply(x):
+        y = torch.zeros_like(x)
+        for d, row in zip(offs, rows):
+            lo, hi = max(0, -d), min(n, n - d)
+            if lo < hi:
+                y[lo:hi] += row[lo + d: hi + d].to(torch.complex128) * x[lo + d: hi + d]
+        return y
+
+    t, want, term = 0.9, psi0.to(torch.complex128), psi0.to(torch.complex128)
+    nrm = torch.linalg.vector_norm(want).item()
+    for k in range(1, 20):
+        term = apply(term) * (-1j * t / k)
+        want = want + term
+    ws = KrylovWorkspace(n, 12, dev)
+    res = expm_krylov(o, v, n, psi0, t, 12, workspace=ws)
+    again = expm_krylov(o, v, n, psi0, t, 12, workspace=ws)
+    assert torch.equal(res.psi, again.psi) and np.array_equal(res.alpha, again.alpha)
+    assert abs(res.psi0_norm - nrm) <= 1e-12 * nrm
+    err = torch.linalg.vector_norm(res.psi.to(torch.complex128) - want).item()
+    assert err <= 2e-6 * nrm, err / nrm
+    # one and two steps: alpha_1 = <psi|H|psi> / <psi|psi>, beta_1 likewise
+    p = psi0.to(torch.complex128)
+    hp = apply(p)
+    a1 = (torch.vdot(p, hp).real / nrm ** 2).item()
+    b1 = torch.linalg.vector_norm(hp - a1 * p).item() / nrm
+    for m in (1, 2):
+        r = expm_krylov(o, v, n, psi0, t, m, workspace=ws)
+        assert r.steps == m
+        assert abs(r.alpha[0] - a1) <= 1e-6 and abs(r.beta[0] - b1) <= 1e-6
+
+
+def test_propagator_from_two_threads(dev):
+    """Calls that overlap on two streams of one process each give the result of
+    a call alone (to rounding: one of them may take the launches per step)."""
+    import threading
+    rng = np.random.default_rng(12)
+    n = 20000
+    offs, vals = [64, 1, 0, -1, -64], []
+    d0 = rng.uniform(-1, 1, n).astype(np.float32)
+    for d in offs:
+        v = np.full(n, -0.5, np.float32) if d else d0.copy()
+        if d > 0:
+            v[:d] = 0
+        elif d < 0:
+            v[n + d:] = 0
+        vals.append(v)
+    o = torch.tensor(offs, dtype=torch.int32, device=dev)
+    v = torch.as_tensor(np.concatenate(vals), device=dev)
+    psi = [torch.as_tensor(_cx(rng, n), device=dev) for _ in range(2)]
+    want = [expm_krylov(o, v, n, p, 0.5, 20).psi.clone() for p in psi]
+    torch.cuda.synchronize()
+    got, failed = [[], []], []
+
+    def work(i):
+        try:
+            st = torch.cuda.Stream()
+            with torch.cuda.stream(st):
+                ws = KrylovWorkspace(n, 20, dev)
+                for _ in range(20):
+                    got[i].append(expm_krylov(o, v, n, psi[i], 0.5, 20, workspace=ws).psi)
+                st.synchronize()
+        except Exception as e:      # reported by the main thread
+            failed.append(e)
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for th in ts:
+        th.start()
+    for th in ts:
+        th.join()
+    assert not failed, failed
+    for i in range(2):
+        for r in got[i]:
+            err = torch.linalg.vector_norm(r - want[i]) / torch.linalg.vector_norm(want[i])
+            assert err.item() <= 2e-6
+
+
 def test_propagator_zero_time_and_zero_state(dev):
     rng = np.random.default_rng(9)
     n = 4097
