@@ -360,7 +360,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_astat(
     const int32_t* __restrict__ C_len, const int64_t* __restrict__ C_starts, int32_t nC,
     const int64_t* __restrict__ pair_ptr, const int4* __restrict__ records,
     const int32_t* __restrict__ aext, T* __restrict__ Cv, int32_t blocks, int32_t groups,
-    int32_t per_xcd, int32_t tail5, T alpha, T sigma)
+    int32_t per_xcd, int32_t chunk, int32_t tail5, T alpha, T sigma)
 {
     // A's smallest and largest offset (written by diagpu_spgemm_astat_prepare
     // after the records)
@@ -372,11 +372,13 @@ __global__ __launch_bounds__(64 * kWaves) void k_astat(
     extern __shared__ float A_l[];   // [nA][kStage] elements: rows i0 - kLead .. i0 + kRB - 1
     const T* A_t = reinterpret_cast<const T*>(A_l);
     // workgroup b on XCD b mod 8: each XCD owns a contiguous range of work
-    // units, so neighbouring blocks (whose B windows overlap) share its L2.
+    // units, so neighbouring blocks (whose B windows overlap) share its L2;
+    // or, with `chunk`, every eighth run of `chunk` units (launch_rows).
     // Unit = (block, group): a block's C diagonals are split over `groups`
     // workgroups (more than one only when the blocks alone cannot fill the
     // GPU), each staging the block's A rows.
-    const int unit = (int)(blockIdx.x % kNumXcd) * per_xcd + (int)(blockIdx.x / kNumXcd);
+    const int xcd = (int)(blockIdx.x % kNumXcd), at = (int)(blockIdx.x / kNumXcd);
+    const int unit = chunk ? (at / chunk * kNumXcd + xcd) * chunk + at % chunk : xcd * per_xcd + at;
     if (unit >= blocks * groups) return;
     // with tail5 the last block (R + 1 rows per lane) goes first: dispatched
     // with the first wave of workgroups, its longer work overlaps the others'
@@ -644,10 +646,21 @@ int launch_rows(const char* fn, int32_t n, const int32_t* A_off, const int64_t* 
     // +-512..+-8192 at n = 2^18..2^20 (forced, one buffer set): 4 -> 16
     // rounds 4-8% faster (config 5: 2.49 -> 2.34 ms under the bench's
     // rotation), 8 -> 16 rounds 3%, at 16 rounds no split gained more than
-    // noise but one (128 x 16 at 2^20, 6%).  Lost with it: complex values
-    // (config 5 complex, 8 rounds: 6.13 -> 6.28 ms at G = 2) and the 8 rows
-    // per lane of the Taylor chain's products (numeric 1.96 -> 2.05 ms).
+    // noise but one (128 x 16 at 2^20, 6%).  Lost with it: complex values at
+    // 2 rows per lane (config 5 complex, 8 rounds: 6.13 -> 6.28 ms at G = 2)
+    // and the 8 rows per lane of the Taylor chain's products (numeric 1.96 ->
+    // 2.05 ms).  Complex values at 4 rows per lane take G = 2 from 100 C
+    // diagonals up to 3 rounds (us, G = 1 -> 2): 5 x 120 and 9 x 100 random
+    // diagonals at n = 150000 185 -> 150 and 242 -> 197, 36 x 60 492 -> 449;
+    // the 7-point stencil times its 63 and 129 diagonals at n = 151951 60.0 ->
+    // 55.4 and 122 -> 105.  Above that 2 % either way (604800: 306 -> 317, 10^6
+    // 541 -> 529), and it loses on short lists (25 C diagonals at 10^6: 49 ->
+    // 66, 63 at 604800: 83.5 -> 85.8).
     int64_t G = 1;
+    if constexpr (sizeof(T) == 8 && R == 4)
+        if (c_ndiag >= 100 &&
+            ceil_div<int64_t>(ceil_div<int64_t>((int64_t)n + kLead, kRB), slots) <= 3)
+            G = 2;
     if constexpr (sizeof(T) == 4 && R == 4) {
         const int64_t r0 = ceil_div<int64_t>(ceil_div<int64_t>((int64_t)n + kLead, kRB), slots);
         while (G < 4 && r0 * G < 16 && c_ndiag >= 2 * G * kPrefetchDiagsPerWave * kWaves) G *= 2;
@@ -676,7 +689,23 @@ int launch_rows(const char* fn, int32_t n, const int32_t* A_off, const int64_t* 
         groups = g5;
         tail5 = 1;
     }
-    const int32_t per_xcd = (int32_t)ceil_div<int64_t>(blocks * groups, kNumXcd);
+    int32_t per_xcd = (int32_t)ceil_div<int64_t>(blocks * groups, kNumXcd);
+    // XCDs interleaved in runs of 4 blocks (8 rows per lane) where C alone is
+    // several times the memory-side cache: with a range of n / 8 rows each,
+    // the XCDs' windows on B lie so far apart that together they exceed that
+    // cache, and a row block's B rows are fetched again for the entries of
+    // the far A offsets.  (us: the 7-point stencil times its 231 and 129
+    // diagonals, 128 x 128 x 64 sites 845 -> 774 and 469 -> 447, 101 x 99 x 105
+    // sites 849 -> 820 and 490 -> 466.  Smaller C loses what neighbouring
+    // blocks share in an XCD's L2: 377 C diagonals at n = 409600 337 -> 345,
+    // 63 at 10^6 65 -> 90.)
+    int32_t chunk = 0;
+    if constexpr (sizeof(T) == 4 && R == 8) {
+        if (n_pairs >= 3 * c_ndiag && c_ndiag * (int64_t)n >= 225000000) {
+            chunk = (int32_t)(4 * groups);
+            per_xcd = (int32_t)(ceil_div<int64_t>(per_xcd, chunk) * chunk);
+        }
+    }
     // the metadata prefetch pays where waves walk many diagonals (config 5:
     // ~575 each) and costs where they walk one or two (the 7-point stencil's
     // square: 25 C diagonals over 16 waves, 31 -> 34 us)
@@ -702,7 +731,7 @@ int launch_rows(const char* fn, int32_t n, const int32_t* A_off, const int64_t* 
         hipLaunchKernelGGL((k_astat<T, kPf, R, kQd, kEp>), grid, block, lds, as_stream(stream), n,
                            A_off, A_starts, nA, A_vals, B_vals, C_off, C_len, C_starts,
                            (int32_t)c_ndiag, pair_ptr, rec, aext, C_vals, (int32_t)blocks,
-                           (int32_t)groups, per_xcd, tail5, alpha, sigma);
+                           (int32_t)groups, per_xcd, chunk, tail5, alpha, sigma);
         return check_launch(fn);
     };
     using yes = std::true_type;
@@ -770,8 +799,16 @@ int launch_astat(const char* fn, int32_t n, const int32_t* A_off, const int64_t*
         if (c_ndiag <= 4 * kWaves && n_pairs <= 4 * c_ndiag && nA <= Astat<T, 16>::kMax &&
             rounds_ok(16, astat_slots<T, 16>(nA)))
             return DIAGPU_ASTAT_LAUNCH(16);
-        // many C diagonals: 8, where two workgroups still fit a CU
-        if (c_ndiag > 4 * kWaves && nA <= Astat<T, 8>::kMax2 && rounds_ok(8, astat_slots<T, 8>(nA)))
+        // many C diagonals: 8, where two workgroups still fit a CU, from 4
+        // rounds, or from n = 100000 where the C diagonals average 3 entries
+        // (us, 4 rows -> 8: the 7-point stencil times its 63, 129 and 231
+        // diagonals at n = 604800 113 -> 90, 303 -> 277, 557 -> 482, at 409600
+        // 78 -> 67, 152 -> 138, 371 -> 337, at 151951 30 -> 28, 51.4 -> 51.1,
+        // 102 -> 89, at 27000 7.9 -> 8.1, 11.3 -> 11.7; plans of about one
+        // entry per C diagonal lose: 5 x 120 at n = 150000 71 -> 79, 400000 177
+        // -> 224)
+        if (c_ndiag > 4 * kWaves && nA <= Astat<T, 8>::kMax2 &&
+            (rounds_ok(8, astat_slots<T, 8>(nA)) || (n >= 100000 && n_pairs >= 3 * c_ndiag)))
             return DIAGPU_ASTAT_LAUNCH(8);
     } else if constexpr (kForceR == 0) {
         // complex: 8 where every wave has at most one C diagonal

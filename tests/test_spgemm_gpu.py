@@ -991,3 +991,36 @@ def test_full_only_for_contiguous_bands_in_order(dev):
         plan.multiply(A.values, A.values, kernel="full")
     assert torch.equal(plan.multiply(A.values, A.values),
                        plan.multiply(A.values, A.values, kernel="gather"))
+
+
+# Launch shapes of the A-stationary kernel: 8 rows per lane from n = 100000 for
+# plans of at least 3 entries per C diagonal, complex values split over two
+# workgroups per block from 100 C diagonals, and XCDs interleaved in runs of 4
+# blocks where C holds 225 million values (1000003 rows: the last run partly
+# empty).  The operand S is the stencil's power S = (I + H)^k on an nx x ny
+# plane, k steps wide.  Bits of the gather.
+@pytest.mark.parametrize("n,nx,ny,k,dtype", [
+    (99999, 40, 50, 3, torch.float32), (100000, 40, 50, 3, torch.float32),
+    (150001, 33, 77, 4, torch.float32), (12345, 17, 23, 3, torch.complex64),
+    (70001, 33, 47, 3, torch.complex64), (200003, 33, 47, 3, torch.complex64),
+    (1000003, 101, 99, 4, torch.float32)])
+def test_astat_launch_shapes_same_bits(dev, n, nx, ny, k, dtype):
+    h = [0, 1, -1, nx, -nx, nx * ny, -nx * ny]
+    s = {0}
+    for _ in range(k):
+        s = {a + b for a in s for b in h}
+    A = workloads.hm_random(n, h, seed=n, device=dev)
+    B = workloads.hm_random(n, s, seed=n + 1, device=dev)
+    av, bv = A.values, B.values
+    if dtype == torch.complex64:
+        av = torch.complex(av, torch.roll(av, 3)).contiguous()
+        bv = torch.complex(bv, torch.roll(bv, 5)).contiguous()
+    plan = SpgemmPlan(A, B)
+    assert plan.info.c_ndiag >= 100 and plan.info.n_pairs >= 3 * plan.info.c_ndiag
+    if n > 10 ** 6:
+        assert plan.info.c_ndiag * n >= 225000000
+    assert plan.kernel_for(dtype) == "astat"
+    word = lambda v: torch.view_as_real(v).view(torch.int32) if v.is_complex() else v.view(torch.int32)
+    C = torch.full((plan.info.c_nnz,), float("nan"), dtype=dtype, device=dev)
+    plan.numeric(av, bv, C, kernel="astat")
+    assert torch.equal(word(C), word(plan.multiply(av, bv, kernel="gather")))
