@@ -72,6 +72,13 @@ class SpgemmInfo(C.Structure):
                 ("b_extent", C.c_int64)]
 
 
+class ChainStep(C.Structure):
+    _fields_ = [("c_ndiag", C.c_int64), ("c_nnz", C.c_int64), ("n_pairs", C.c_int64),
+                ("max_pairs", C.c_int64), ("b_extent", C.c_int64), ("c_off", C.c_int64),
+                ("c_len", C.c_int64), ("c_starts", C.c_int64), ("pair_ptr", C.c_int64),
+                ("records", C.c_int64), ("has_main", C.c_int32), ("b_in_range", C.c_int32)]
+
+
 class SpgemmShape(C.Structure):
     _fields_ = [("a_off_min", C.c_int32), ("a_off_max", C.c_int32), ("b_off_min", C.c_int32),
                 ("b_off_max", C.c_int32), ("contiguous", C.c_int32)]
@@ -123,6 +130,8 @@ PROTOTYPES: dict[str, tuple] = {
         _vp, _sz,
         _vp, C.POINTER(_i32), C.POINTER(SpgemmShape),
         C.POINTER(SpgemmInfo), _vp]),
+    "diagpu_chain_plans": (C.c_int, [_i32, _i32, _vp, _i32, _vp, _i32, _vp, _sz, C.POINTER(_sz),
+                                     C.POINTER(ChainStep)]),
     "diagpu_spgemm_full_choice": (C.c_int, [_i32, _i32, _i32, _i64, _i64, C.POINTER(SpgemmShape),
                                             _i32]),
     "diagpu_spgemm_numeric_full_f32": (C.c_int, [_i32, _i32, _i32, _vp, _vp, _i32, _i32, _vp, _vp,

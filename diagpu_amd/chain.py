@@ -3,9 +3,11 @@ of the SpGEMM hot path that the reference describes but does not ship
 (spmspm/gather_flat.cuh:13-14 "recurs each step of a matrix-power chain where
 A grows"; :110-117 "fully on-device plan build").
 
-Every product builds its C structure and pair plan on the GPU
-(diagpu_spgemm_symbolic; one stream sync returns the counts) and fills C with
-diagpu_spgemm_numeric_f32 (or _c64).  Sums and scalings use
+A product builds its C structure and pair plan on the GPU
+(diagpu_spgemm_symbolic_shape; one stream sync returns the counts) and fills C
+with diagpu_spgemm_numeric_f32 (or _c64).  A chain's products after the first
+are planned on the host from the offsets, all in one call
+(diagpu_chain_plans), and run without a wait between them.  Sums and scalings use
 diagpu_dia_axpby_f32 (or _c64) over the union of the operands' diagonals; the
 union itself is a merge of two short sorted offset lists on the host.  A
 Taylor step I + ((t/j) H) S whose plan the A-stationary kernel takes is one
@@ -20,6 +22,7 @@ torch tensors only carry device memory; all arithmetic is in libdiagpu.
 """
 from __future__ import annotations
 
+import ctypes
 import time
 from dataclasses import dataclass, field
 
@@ -27,7 +30,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .spgemm import SpgemmPlan, _check_dev
+from .spgemm import BAND_LDS_BUDGET, BAND_ROWS, SpgemmPlan, _check_dev
 from .spmv import _on_stream, _stream_handle
 from .workloads import HM, hm_layout
 
@@ -242,6 +245,93 @@ def _narrow_first(X: HM) -> bool:
     return X.values.dtype == torch.float32 or X.ndiag <= _lib.ASTAT_MAX_A_C64
 
 
+class _HostPlans:
+    """The products C_t = H C_{t-1}, t = 1 .. steps, C_0 on the diagonals
+    `first`, planned on the host in one call (diagpu_chain_plans) and copied
+    to the device together: no read-back between the products.  `ok` is False
+    where a product is not the A-stationary kernel's (then the device plans
+    its products)."""
+
+    def __init__(self, H: HM, first: list[int], steps: int):
+        self.H, self.n = H, H.n
+        ho = _host_offsets(H)
+        dt = H.values.dtype
+        cap = _lib.ASTAT_MAX_A if dt == torch.float32 else _lib.ASTAT_MAX_A_C64
+        self.ok = 4096 <= H.n < 1 << 30 and 1 <= len(ho) <= cap and len(first) > 0
+        if not self.ok:
+            return
+        ha, sa = np.asarray(ho, np.int32), np.asarray(first, np.int32)
+        self.steps = (_lib.ChainStep * steps)()
+        need = ctypes.c_size_t(1 << 17)
+        while True:
+            host = torch.empty(need.value, dtype=torch.uint8, pin_memory=True)
+            st = _lib.load().diagpu_chain_plans(
+                H.n, len(ho), ha.ctypes.data, len(first), sa.ctypes.data, steps, host.data_ptr(),
+                host.numel(), ctypes.byref(need), self.steps)
+            if st != _lib.ERR_CAPACITY or need.value <= host.numel():
+                break
+        if st != _lib.OK:       # a long chain, or offsets in another order: the device plans
+            self.ok = False
+            return
+        self.host = host
+        self.stream = torch.cuda.current_stream(H.values.device).cuda_stream
+        nb = len(first)
+        for s in self.steps:
+            self.ok = self.ok and bool(s.b_in_range) and self._astat(ho, nb, s, dt)
+            nb = s.c_ndiag
+        if self.ok:
+            self.buf = torch.empty(need.value, dtype=torch.uint8, device=H.values.device)
+            self.buf.copy_(host[: need.value], non_blocking=True)
+            self.base = self.buf.data_ptr()
+
+    def _astat(self, ho, nb: int, s, dt) -> bool:
+        """Whether SpgemmPlan's choice for step s is the A-stationary kernel
+        (uses_band, uses_full and uses_astat, from the host's counts; plans
+        that may be one of the others' are left to the device path)."""
+        na, np_, nc = len(ho), s.n_pairs, s.c_ndiag
+        if nc == 0 or nc >= 1 << 29 or np_ >= 1 << 28 or np_ == na * nb and nc == na + nb - 1:
+            return False
+        if dt == torch.complex64:
+            return self.n >= 1 << 16 or np_ >= 3 * na
+        if np_ >= 3 * nc and self.n >= 1024 * BAND_ROWS:
+            wb = (BAND_ROWS + ho[-1] - ho[0] + 3) & ~3
+            if 4 * (na * BAND_ROWS + nb * wb) + 16 * np_ <= BAND_LDS_BUDGET:
+                return False
+        return not (np_ < 16 and 2 * np_ >= 3 * nc and 1 << 19 <= self.n < 1 << 20)
+
+    def product(self, t: int, B: torch.Tensor, alpha=None, sigma=0.0) -> torch.Tensor:
+        """C_t's values from C_{t-1}'s: H B, or (alpha H) B + sigma I."""
+        H, s, b = self.H, self.steps[t - 1], self.base
+        if B.numel() < s.b_extent:
+            raise ValueError(f"B holds {B.numel()} values, the product needs {s.b_extent}")
+        Cv = _c_values(s.c_nnz, H.values)
+        real = H.values.dtype == torch.float32
+        head = (H.n, H.offsets.data_ptr(), H.starts.data_ptr(), H.ndiag, H.values.data_ptr())
+        tail = (B.data_ptr(), b + s.c_off, b + s.c_len, b + s.c_starts, s.c_ndiag, b + s.pair_ptr,
+                b + s.records, s.n_pairs)
+        if alpha is None:
+            _lib.call("diagpu_spgemm_numeric_astat_f32" if real
+                      else "diagpu_spgemm_numeric_astat_c64", *head, *tail, Cv.data_ptr(),
+                      self.stream)
+        else:
+            a, sg = (float(alpha), float(sigma)) if real else (_c64(alpha), _c64(sigma))
+            _lib.call("diagpu_spgemm_numeric_astat_scaled_f32" if real
+                      else "diagpu_spgemm_numeric_astat_scaled_c64", *head, a, *tail, sg,
+                      Cv.data_ptr(), self.stream)
+        return Cv
+
+    def result(self, values: torch.Tensor) -> HM:
+        """The last step's C (its structure views of the copied buffer)."""
+        s = self.steps[len(self.steps) - 1]
+
+        def view(at, count, dt, size):
+            return self.buf[at: at + count * size].view(dt)
+        return HM(self.n, view(s.c_off, s.c_ndiag, torch.int32, 4),
+                  view(s.c_len, s.c_ndiag, torch.int32, 4),
+                  view(s.c_starts, s.c_ndiag, torch.int64, 8), values,
+                  self.host[s.c_off: s.c_off + 4 * s.c_ndiag].view(torch.int32).tolist())
+
+
 def power(H: HM, k: int, stats: ChainStats | None = None) -> HM:
     """H^k (k >= 1) by the chain P_j = H * P_{j-1} (P_{j-1} * H for complex
     values when H is too wide for the complex A-stationary kernel; the
@@ -257,12 +347,19 @@ def power(H: HM, k: int, stats: ChainStats | None = None) -> HM:
 
 
 def _power_steps(H: HM, k: int) -> HM:
-    """power() with each product's plan built on the side stream while the
-    previous product runs (as _taylor_steps): a plan needs only the
-    operands' structure, and P_{j-1}'s is the previous plan's C arrays,
-    complete once its symbolic phase has returned.  Products stay on the
-    caller's stream, in order."""
+    """power() without a wait between the products.  The first product is
+    planned on the device, which checks H; the others' plans follow from its
+    offsets on the host (_HostPlans).  Where a product is not the
+    A-stationary kernel's, each plan is built on the side stream while the
+    previous product runs (as _taylor_steps): a plan needs only the operands'
+    structure, and P_{j-1}'s is the previous plan's C arrays, complete once
+    its symbolic phase has returned.  Products stay on the caller's stream, in
+    order."""
     main = torch.cuda.current_stream(H.values.device)
+    plans = None
+    if k >= 3 and _narrow_first(H):
+        ho = _host_offsets(H)
+        plans = _HostPlans(H, _sumset(H.n, ho, ho), k - 2)
     side = _side_stream(H.values.device)
     side.wait_stream(main)                      # H's structure
     narrow = _narrow_first(H)
@@ -281,6 +378,11 @@ def _power_steps(H: HM, k: int) -> HM:
                 plan.numeric(H.values, P.values, C.values)
             else:
                 plan.numeric(P.values, H.values, C.values)
+        if plans is not None and plans.ok:
+            v = C.values
+            for t in range(1, k - 1):
+                v = plans.product(t, v)
+            return plans.result(v)
         C.host_offsets = _sumset(H.n, _host_offsets(H), _host_offsets(P))   # while it runs
         P = C
     return P
@@ -420,17 +522,27 @@ def _side_stream(device) -> torch.cuda.Stream:
 
 
 def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event) -> HM:
-    """The Horner steps of taylor_expm with each product's plan built on a
-    side stream while the previous product runs: a plan needs only its
-    operands' structure (the previous plan's C arrays, complete once its
-    symbolic phase has returned), so its one stream sync waits for its own
-    symbolic phase, not for the product queued before it.  Products,
-    scalings and identity adds stay on the caller's stream, in order.
+    """The Horner steps of taylor_expm without a wait between the products.
+    The first is planned on the device, which checks H; the others' plans
+    follow from its offsets on the host (_HostPlans).  Where a step is not a
+    fused product, each product's plan is built on a side stream while the
+    previous product runs: a plan needs only its operands' structure (the
+    previous plan's C arrays, complete once its symbolic phase has returned),
+    so its one stream sync waits for its own symbolic phase, not for the
+    product queued before it.  Products, scalings and identity adds stay on
+    the caller's stream, in order.
     `ready`: recorded on the caller's stream before S was formed; where S
     shares H's structure, the first plan waits for it only, not for the
     pass that formed S's values."""
     main = torch.cuda.current_stream(H.values.device)
     side = _side_stream(H.values.device)
+    # the steps after the first, planned on the host where they are all fused
+    # products with I on their main diagonals
+    plans = None
+    if order >= 3 and _narrow_first(H):
+        plans = _HostPlans(H, _sumset(H.n, _host_offsets(H), _host_offsets(S)), order - 2)
+        if not (plans.ok and all(s.has_main for s in plans.steps)):
+            plans = None
     if S.offsets is H.offsets and S.starts is H.starts and S.lengths is H.lengths:
         side.wait_event(ready)                  # H's structure
     else:
@@ -458,6 +570,11 @@ def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event) -> HM:
                 else:
                     plan.numeric(S.values, Hj.values, C.values)
             sigma = 0.0
+        if plans is not None and sigma and j == order - 1:
+            v = C.values
+            for t_ in range(1, order - 1):
+                v = plans.product(t_, v, t / (order - 1 - t_), 1.0)
+            return plans.result(v)
         C.host_offsets = _sumset(H.n, _host_offsets(H), _host_offsets(S))   # while the product runs
         S = C if sigma else add_identity(C)
         if S.offsets is not C.offsets:

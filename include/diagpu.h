@@ -406,6 +406,35 @@ DIAGPU_API int diagpu_spgemm_symbolic_astat(
     int32_t* records, int32_t* records_status,
     diagpu_spgemm_info* info, void* stream);
 
+/* One product of a chain planned on the host (diagpu_chain_plans): counts, and
+ * where its arrays start in the buffer (bytes). */
+typedef struct diagpu_chain_step {
+    int64_t c_ndiag, c_nnz, n_pairs, max_pairs;
+    int64_t b_extent;                /* values of the B operand                  */
+    int64_t c_off, c_len, c_starts;  /* int32, int32, int64 [c_ndiag]            */
+    int64_t pair_ptr;                /* int64 [c_ndiag + 1]                      */
+    int64_t records;                 /* int32 [4 n_pairs + 4], as                */
+                                     /* diagpu_spgemm_symbolic_astat's          */
+    int32_t has_main;                /* 1: C holds the main diagonal             */
+    int32_t b_in_range;              /* 1: B indices below 2^30 (else the        */
+                                     /* records are unusable)                    */
+} diagpu_chain_step;
+
+/* Plans of the chain C_t = H C_{t-1}, t = 1 .. steps, C_0 = S, on the host
+ * (no HIP call; every pointer is host memory): the arrays the symbolic phase
+ * builds for H and C_{t-1}, with the A-stationary records, S and every C in
+ * the standard layout (diagonals in offset order, starts the running sum of
+ * the lengths).  Offsets ascending, distinct, inside (-n, n) (else
+ * DIAGPU_ERR_OFFSET).  out of `capacity` bytes (16-byte aligned) receives the
+ * arrays if they fit, else DIAGPU_ERR_CAPACITY with *needed set (capacity 0
+ * asks for it); info[steps] is filled in both cases.  Chains of
+ * more than 32768 offset sums in all are refused with DIAGPU_ERR_OVERFLOW (the
+ * device plans those faster).  No reference counterpart (spmspm/gather_flat.cuh:13-14 describes the chain). */
+DIAGPU_API int diagpu_chain_plans(int32_t n, int32_t h_ndiag, const int32_t* h_offsets,
+                                  int32_t s_ndiag, const int32_t* s_offsets, int32_t steps,
+                                  void* out, size_t capacity, size_t* needed,
+                                  diagpu_chain_step* info);
+
 /* What the symbolic phase saw of the operands' offsets (host memory). */
 typedef struct diagpu_spgemm_shape {
     int32_t a_off_min, a_off_max;   /* smallest and largest A offset            */

@@ -320,3 +320,76 @@ def test_full_argument_errors():
     assert _status(name, 10000, -100, 201, f, f, -1, 3, f, f, f, 203, f, None) == _lib.ERR_CAPACITY
     assert _status("diagpu_spgemm_symbolic_shape", 4, f, f, f, 1, f, f, f, 1, f, f, f, 1, f, f, 1,
                    None, f, 1 << 20, None, None, None, C.byref(_lib.SpgemmInfo()), None) == _lib.ERR_ARG
+
+
+def test_chain_plans_argument_errors():
+    name = "diagpu_chain_plans"
+    off = (C.c_int32 * 3)(-1, 0, 1)
+    bad = (C.c_int32 * 3)(-1, 1, 0)
+    need, info = C.c_size_t(0), (_lib.ChainStep * 2)()
+    buf = C.create_string_buffer(1 << 16)
+    ok = (100, 3, off, 3, off, 2, buf, len(buf), C.byref(need), info)
+    assert _status(name, *ok) == _lib.OK and need.value > 0
+    for at, v, code in ((0, 0, _lib.ERR_ARG), (1, 0, _lib.ERR_ARG), (2, None, _lib.ERR_ARG),
+                        (2, bad, _lib.ERR_OFFSET), (4, bad, _lib.ERR_OFFSET), (5, 0, _lib.ERR_ARG),
+                        (6, None, _lib.ERR_ARG), (8, None, _lib.ERR_ARG), (9, None, _lib.ERR_ARG),
+                        (0, 1, _lib.ERR_OFFSET)):
+        args = list(ok)
+        args[at] = v
+        assert _status(name, *args) == code, (at, v)
+    assert _status(name, 100, 3, off, 3, off, 2, None, 0, C.byref(need), info) == _lib.ERR_CAPACITY
+    assert _status(name, 100, 3, off, 3, off, 2, buf, need.value, C.byref(need), info) == _lib.OK
+    assert _status(name, 100, 3, off, 3, off, 2, buf, need.value - 1, C.byref(need),
+                   info) == _lib.ERR_CAPACITY
+    long = (C.c_int32 * 200)(*range(-100, 100))
+    big = (_lib.ChainStep * 1)()
+    assert _status(name, 9000, 200, long, 200, long, 1, None, 0, C.byref(need),
+                   big) == _lib.ERR_OVERFLOW
+
+
+@pytest.mark.parametrize("n,h,s,steps", [
+    (10, [0], [0], 3), (10, [-9, 9], [-9, 9], 2), (50, [-7, -1, 0, 1, 7], [-7, 0, 3], 4),
+    (40, [-13, 2, 5], [-39, -20, 0, 38], 5), (9, [-3, 1, 4], [-8, -2, 0, 5, 8], 6),
+    (5000, [-300, -17, -1, 0, 1, 17, 300], [-300, -17, -1, 0, 1, 17, 300], 4),
+    (100000, [5, 90000], [-99999, -5, 7], 3)])
+def test_chain_plans_match_the_reference_planners(oracle, n, h, s, steps):
+    """Every array against the oracle's restatement of the reference planners:
+    C structure, pair_ptr, and each record against its GPair (A index, range
+    of C positions where both operands hold an element, B index of position 0)."""
+    import numpy as np
+    ha, sa = np.array(h, np.int32), np.array(s, np.int32)
+    info, need = (_lib.ChainStep * steps)(), C.c_size_t(0)
+    fn = _lib.load().diagpu_chain_plans
+    args = (n, len(h), ha.ctypes.data, len(s), sa.ctypes.data, steps)
+    assert fn(*args, None, 0, C.byref(need), info) == _lib.ERR_CAPACITY
+    buf = np.zeros(need.value, np.uint8)
+    assert fn(*args, buf.ctypes.data, buf.size, C.byref(need), info) == _lib.OK
+    at = lambda o, c, dt: buf[o: o + c * np.dtype(dt).itemsize].view(dt)
+    layout = lambda o: (o, (n - np.abs(o.astype(np.int64))).astype(np.int32))
+    starts = lambda ln: np.concatenate([[0], np.cumsum(ln.astype(np.int64))[:-1]])
+    a_off, a_len = layout(ha)
+    a_st = starts(a_len)
+    b_off = sa
+    for t in range(steps):
+        b_off, b_len = layout(b_off)
+        b_st = starts(b_len)
+        c_off, c_len, c_st, nnz = oracle.c_structure(n, a_off, b_off)
+        ptr, pairs = oracle.pairs_only(n, a_off, a_len, a_st, b_off, b_len, b_st, c_off)
+        x = info[t]
+        assert (x.c_ndiag, x.c_nnz, x.n_pairs) == (len(c_off), nnz, ptr[-1])
+        assert x.max_pairs == np.diff(ptr).max() and x.b_extent == b_len.sum()
+        assert x.has_main == (0 in c_off) and x.b_in_range == 1
+        assert np.array_equal(at(x.c_off, x.c_ndiag, np.int32), c_off)
+        assert np.array_equal(at(x.c_len, x.c_ndiag, np.int32), c_len)
+        assert np.array_equal(at(x.c_starts, x.c_ndiag, np.int64), c_st)
+        assert np.array_equal(at(x.pair_ptr, x.c_ndiag + 1, np.int64), ptr)
+        rec = at(x.records, 4 * x.n_pairs + 4, np.int32)
+        r = rec[:-4].reshape(-1, 4)
+        lo = np.maximum(0, np.maximum(-pairs["ash"], -pairs["bsh"]))
+        hi = np.minimum(pairs["al"] - pairs["ash"], pairs["bl"] - pairs["bsh"])
+        assert (lo < hi).all()
+        assert np.array_equal(a_st[r[:, 0]], pairs["ab"].astype(np.int64))
+        assert np.array_equal(r[:, 1], lo) and np.array_equal(r[:, 2], hi)
+        assert np.array_equal(r[:, 3], pairs["bb"].astype(np.int64) + pairs["bsh"])
+        assert rec[-4:].tolist() == [0, 0, h[0], h[-1]]
+        b_off = c_off

@@ -17,7 +17,7 @@ import pytest
 import scipy.linalg
 import torch
 
-from diagpu_amd import chain
+from diagpu_amd import chain, workloads
 from diagpu_amd.workloads import HM, hm_random, hm_stencil7
 from hm_host import dense_of, matvec64
 
@@ -375,3 +375,51 @@ def test_power_pipelined_matches_synced(dev, complex_values):
     torch.cuda.synchronize()
     assert P1.offsets.cpu().tolist() == P2.offsets.cpu().tolist() == P1.host_offsets
     assert torch.equal(P1.values.view(torch.int32), P2.values.view(torch.int32))
+
+
+# The chains whose later products are planned on the host, against the same
+# chain with every product planned on the device (the timed form, `stats`):
+# the same structure and the same bits.  Lattices whose products hold the main
+# diagonal; one-sided diagonals, which never do; a chain too long for the host
+# planner; n below the A-stationary kernel; a contiguous band.
+@pytest.mark.parametrize("n,offs", [
+    (4096, [-64, -1, 0, 1, 64]), (20011, [-900, -30, -1, 0, 1, 30, 900]),
+    (140000, [-900, -30, -1, 0, 1, 30, 900]), (9001, [1, 40, 300]), (4095, [-64, -1, 0, 1, 64]),
+    (30000, [-1, 0, 1]), (50000, [-9000, 0, 8000]), (6000, list(range(-300, 300, 23)))])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_host_planned_chain_same_bits(dev, n, offs, cplx):
+    H = workloads.hm_random(n, offs, seed=n, device=dev)
+    t = 0.3 - 0.2j if cplx else 0.3
+    word = lambda v: torch.view_as_real(v).view(torch.int32) if v.is_complex() else v.view(torch.int32)
+
+    def same(x, y):
+        assert torch.equal(x.offsets, y.offsets) and torch.equal(x.starts, y.starts)
+        assert torch.equal(x.lengths, y.lengths)
+        assert torch.equal(word(x.values), word(y.values))
+        assert x.host_offsets == x.offsets.cpu().tolist()
+
+    for order in (2, 3, 5):
+        same(chain.taylor_expm(H, t, order), chain.taylor_expm(H, t, order, chain.ChainStats()))
+    G = chain.as_complex(H) if cplx else H
+    for k in (2, 3, 4):
+        same(chain.power(G, k), chain.power(G, k, chain.ChainStats()))
+
+
+def test_chain_still_refuses_wrong_lengths(dev):
+    from diagpu_amd import _lib
+    H = workloads.hm_random(5000, [-70, -1, 0, 1, 70], seed=3, device=dev)
+    H.lengths = H.lengths - 1
+    with pytest.raises(_lib.DiagpuError):
+        chain.power(H, 4)
+    with pytest.raises(_lib.DiagpuError):
+        chain.taylor_expm(H, 0.1, 4)
+
+
+def test_power_of_unordered_offsets(dev):
+    """Offsets in descending order: planned on the device, as before."""
+    A = workloads.hm_random(5000, [-70, -1, 0, 1, 70], seed=4, device=dev)
+    R = workloads.HM(A.n, A.offsets.flip(0).contiguous(), A.lengths.flip(0).contiguous(),
+                     A.starts.flip(0).contiguous(), A.values)
+    x, y = chain.power(R, 4), chain.power(A, 4)
+    assert torch.equal(x.offsets, y.offsets)
+    assert torch.allclose(x.values, y.values, rtol=0, atol=1e-4)
