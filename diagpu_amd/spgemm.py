@@ -32,6 +32,16 @@ BAND_ROWS = 256
 BAND_LDS_BUDGET = 64 * 1024
 
 
+# value dtype -> numeric entry points: gather, A-stationary, contiguous band
+_NUMERIC = {
+    torch.float32: ("diagpu_spgemm_numeric_f32", "diagpu_spgemm_numeric_astat_f32",
+                    "diagpu_spgemm_numeric_full_f32"),
+    torch.complex64: ("diagpu_spgemm_numeric_c64", "diagpu_spgemm_numeric_astat_c64",
+                      "diagpu_spgemm_numeric_full_c64"),
+}
+_KERNELS = frozenset(("auto", "gather", "band", "astat", "full", "band_mfma"))
+
+
 class SpgemmPlan:
     """C = A * B for HM operands (objects with n, offsets, lengths, starts,
     int32/int32/int64 device tensors).  Builds the C structure and pair plan
@@ -75,12 +85,13 @@ class SpgemmPlan:
             self._parts[name] = (o, dt, cnt, esz[dt])
             o += sz
         self._base = self._buf.data_ptr()
+        self._at = {name: self._base + v[0] for name, v in self._parts.items()}
         self.info = _lib.SpgemmInfo()
         self._band = None
         self._astat = None
         self._rstat = C.c_int32(0)
         self.shape = _lib.SpgemmShape()
-        self._full = {}
+        self._full, self._auto = {}, {}
         self._sym_fn = _lib.load().diagpu_spgemm_symbolic_shape
         self._sym_args, self._sym_caps, self._sym_ops = None, None, ()
         self.symbolic()
@@ -95,7 +106,7 @@ class SpgemmPlan:
         return v
 
     def _addr(self, name: str):
-        return self._base + self._parts[name][0] if name in self._parts else None
+        return self._at.get(name)
 
     C_off = property(lambda self: self._view("C_off"))
     C_len = property(lambda self: self._view("C_len"))
@@ -112,7 +123,7 @@ class SpgemmPlan:
         sync)."""
         self._band = None
         self._astat = None
-        self._full = {}
+        self._full, self._auto = {}, {}
         A, B = self.A, self.B
         ops = (A.offsets, A.lengths, A.starts, B.offsets, B.lengths, B.starts)
         if (self._sym_caps != (self.c_cap, self.p_cap)
@@ -135,6 +146,8 @@ class SpgemmPlan:
                                C.byref(self.info))
             self._sym_caps = (self.c_cap, self.p_cap)
         st = self._sym_fn(*self._sym_args, _stream_handle(self.stream))
+        inf = self.info
+        self._counts = (inf.c_ndiag, inf.c_nnz, inf.n_pairs, inf.a_extent, inf.b_extent)
         if st:
             _lib.check(st)
         if self._fused:
@@ -360,33 +373,37 @@ class SpgemmPlan:
         "band_mfma" (fp32, narrow bands on the matrix cores: the same values
         to rounding, finite operands)."""
         dt = A_vals.dtype
-        name = {torch.float32: "diagpu_spgemm_numeric_f32",
-                torch.complex64: "diagpu_spgemm_numeric_c64"}.get(dt)
-        if name is None:
+        names = _NUMERIC.get(dt)
+        if names is None:
             raise TypeError(f"unsupported value dtype {dt}")
-        if kernel not in ("auto", "gather", "band", "astat", "full", "band_mfma"):
+        if kernel not in _KERNELS:
             raise ValueError(f"unknown kernel {kernel!r}")
         _check_dev(A_vals, dt, "A_vals")
         _check_dev(B_vals, dt, "B_vals")
         _check_dev(C_vals, dt, "C_vals")
-        if A_vals.numel() < self.info.a_extent or B_vals.numel() < self.info.b_extent:
+        c_ndiag, c_nnz, n_pairs, a_extent, b_extent = self._counts
+        if A_vals.numel() < a_extent or B_vals.numel() < b_extent:
             raise ValueError(f"A_vals / B_vals hold {A_vals.numel()} / {B_vals.numel()} values; "
-                             f"the plan's operands need {self.info.a_extent} / "
-                             f"{self.info.b_extent}")
-        if C_vals.numel() < self.info.c_nnz:
-            raise ValueError(f"C_vals has {C_vals.numel()} elements, needs {self.info.c_nnz}")
+                             f"the plan's operands need {a_extent} / {b_extent}")
+        if C_vals.numel() < c_nnz:
+            raise ValueError(f"C_vals has {C_vals.numel()} elements, needs {c_nnz}")
         if kernel == "auto":
-            kernel = "full" if self.uses_full(dt) else self.kernel_for(dt)
+            kernel = self._auto.get(dt)
+            if kernel is None:
+                kernel = "full" if self.uses_full(dt) else self.kernel_for(dt)
+                self._auto[dt] = kernel
+        lib = _lib.load()
         if kernel == "full":
             if not self.shape.contiguous:
                 raise ValueError("the full kernel takes contiguous bands in ascending order")
             A, B = self.A, self.B
-            _lib.call("diagpu_spgemm_numeric_full_f32" if dt == torch.float32
-                      else "diagpu_spgemm_numeric_full_c64", self.n, self.shape.a_off_min,
-                      A.offsets.numel(), A.starts.data_ptr(), A_vals.data_ptr(),
-                      self.shape.b_off_min, B.offsets.numel(), B.starts.data_ptr(),
-                      B_vals.data_ptr(), self._addr("C_starts"), self.info.c_ndiag,
-                      C_vals.data_ptr(), _stream_handle(self.stream))
+            st = getattr(lib, names[2])(
+                self.n, self.shape.a_off_min, A.offsets.numel(), A.starts.data_ptr(),
+                A_vals.data_ptr(), self.shape.b_off_min, B.offsets.numel(), B.starts.data_ptr(),
+                B_vals.data_ptr(), self._at["C_starts"], c_ndiag, C_vals.data_ptr(),
+                _stream_handle(self.stream))
+            if st:
+                _lib.check(st)
             return
         if kernel in ("band", "band_mfma") and dt != torch.float32:
             raise TypeError(f"the {kernel} kernel is fp32")
@@ -401,15 +418,15 @@ class SpgemmPlan:
                       _stream_handle(self.stream))
             return
         if kernel == "astat":
-            rec = (self._addr("records") if self._astat is True
-                   else self.astat_records().data_ptr())
+            at = self._at
+            rec = at["records"] if self._astat is True else self.astat_records().data_ptr()
             A = self.A
-            _lib.call("diagpu_spgemm_numeric_astat_f32" if dt == torch.float32
-                      else "diagpu_spgemm_numeric_astat_c64", self.n, A.offsets.data_ptr(),
-                      A.starts.data_ptr(), A.offsets.numel(), A_vals.data_ptr(), B_vals.data_ptr(),
-                      self.C_off.data_ptr(), self.C_len.data_ptr(), self.C_starts.data_ptr(),
-                      self.info.c_ndiag, self.ptr.data_ptr(), rec, self.info.n_pairs,
-                      C_vals.data_ptr(), _stream_handle(self.stream))
+            st = getattr(lib, names[1])(
+                self.n, A.offsets.data_ptr(), A.starts.data_ptr(), A.offsets.numel(),
+                A_vals.data_ptr(), B_vals.data_ptr(), at["C_off"], at["C_len"], at["C_starts"],
+                c_ndiag, at["ptr"], rec, n_pairs, C_vals.data_ptr(), _stream_handle(self.stream))
+            if st:
+                _lib.check(st)
             return
         if kernel == "band":
             pab, info = self.band_info()
@@ -421,7 +438,7 @@ class SpgemmPlan:
                       self.info.c_ndiag, self.ptr.data_ptr(), pab.data_ptr(), C.byref(info),
                       C_vals.data_ptr(), _stream_handle(self.stream))
             return
-        st = getattr(_lib.load(), name)(
+        st = getattr(lib, names[0])(
             self.n, A_vals.data_ptr(), B_vals.data_ptr(), self.C_off.data_ptr(),
             self.C_len.data_ptr(), self.C_starts.data_ptr(), self.info.c_ndiag,
             self.ptr.data_ptr(), self.pairs.data_ptr(), self.info.max_pairs,

@@ -27,16 +27,23 @@ def _on_stream(stream):
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _stream_handle(stream) -> int:
+    """The raw handle of `stream`, or of the current stream (the caller holds
+    device tensors, so the device is initialised)."""
     if stream is None:
-        if _raw_stream is not None:      # the current stream's handle, without a Stream object
-            return _raw_stream(torch.cuda.current_device())
+        if _raw_stream is not None and _raw_device is not None:   # without a Stream object
+            return _raw_stream(_raw_device())
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
     return int(stream)
+
+
+_VIEWS = {torch.float32: _lib.ReconViewF32, torch.float64: _lib.ReconViewF64,
+          torch.complex64: _lib.ReconViewC64}
 
 
 def recon_view(offsets: torch.Tensor, values: torch.Tensor, rows: int, cols: int):
@@ -48,8 +55,7 @@ def recon_view(offsets: torch.Tensor, values: torch.Tensor, rows: int, cols: int
     K = offsets.numel()
     if values.numel() != K * cols:
         raise ValueError(f"values has {values.numel()} elements, expected K*cols = {K * cols}")
-    cls = {torch.float32: _lib.ReconViewF32, torch.float64: _lib.ReconViewF64,
-           torch.complex64: _lib.ReconViewC64}.get(values.dtype)
+    cls = _VIEWS.get(values.dtype)
     if cls is None:
         raise TypeError(f"unsupported dtype {values.dtype}")
     return cls(rows, cols, K, offsets.data_ptr(), values.data_ptr())
@@ -78,5 +84,8 @@ def spmv_recon(offsets: torch.Tensor, values: torch.Tensor, rows: int, cols: int
         y = torch.empty(rows, dtype=x.dtype, device=values.device)
     if y.dtype != x.dtype or y.numel() < rows or not y.is_cuda or not y.is_contiguous():
         raise TypeError("y must be a contiguous device tensor of x's dtype with >= rows elements")
-    _lib.call(name, C.byref(view), x.data_ptr(), x.numel(), y.data_ptr(), _stream_handle(stream))
+    st = getattr(_lib.load(), name)(C.byref(view), x.data_ptr(), x.numel(), y.data_ptr(),
+                                    _stream_handle(stream))
+    if st:
+        _lib.check(st)
     return y
