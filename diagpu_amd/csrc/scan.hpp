@@ -8,6 +8,33 @@
 namespace diagpu {
 
 // Inclusive prefix sum across the 64 lanes of a wave.
+// `x` moved between lanes by a DPP control; lanes that get nothing keep `id`.
+template <int Ctrl, int RowMask>
+__device__ __forceinline__ int32_t dpp_move(int32_t x, int32_t id)
+{
+    return __builtin_amdgcn_update_dpp(id, x, Ctrl, RowMask, 0xf, false);
+}
+template <int Ctrl, int RowMask>
+__device__ __forceinline__ int64_t dpp_move(int64_t x, int64_t id)
+{
+    const int32_t lo = dpp_move<Ctrl, RowMask>((int32_t)x, (int32_t)id);
+    const int32_t hi = dpp_move<Ctrl, RowMask>((int32_t)(x >> 32), (int32_t)(id >> 32));
+    return ((int64_t)hi << 32) | (uint32_t)lo;
+}
+
+// Inclusive scan under `op` (identity `id`) over the wave's lanes: within
+// rows of 16 lanes, then across the rows.  Lane 63 holds the wave's result.
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_scan_dpp(T v, T id, Op op)
+{
+    v = op(v, dpp_move<0x111, 0xf>(v, id));   // row_shr:1
+    v = op(v, dpp_move<0x112, 0xf>(v, id));   // row_shr:2
+    v = op(v, dpp_move<0x114, 0xf>(v, id));   // row_shr:4
+    v = op(v, dpp_move<0x118, 0xf>(v, id));   // row_shr:8
+    v = op(v, dpp_move<0x142, 0xa>(v, id));   // row_bcast:15
+    return op(v, dpp_move<0x143, 0xc>(v, id));   // row_bcast:31
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_inclusive_scan(T v)
 {

@@ -56,6 +56,7 @@ constexpr int kFastBlock = 512;
 constexpr int kFastWaves = kFastBlock / 64;
 constexpr int kFastLdsBytes = 128 * 1024;
 constexpr int kFastLdsWords = kFastLdsBytes / 4;
+constexpr int kFastClear = 2048;   // bitmap words cleared before the spans are known
 constexpr int kMaxFastGroups = 1024;
 constexpr int64_t kFastMaxProducts = int64_t(1) << 20;
 
@@ -423,21 +424,23 @@ __global__ __launch_bounds__(kBlock) void k_pair_fill(
 // exchange their totals once, and each wave then writes its diagonals'
 // starts, pair_ptr and GPairs (slot ranks from the same ballot: B order).
 // Everything a workgroup combines goes through one LDS exchange and one
-// barrier per step (eight in all, nine with the A-stationary records).
+// barrier per step.
 // Counts, nnz, useful flops and the operands' value extents are computed by
 // every workgroup and written by workgroup 0; each workgroup writes its
 // largest entry count (wg_max) and, with the records, its flag word (wg_rec),
 // and the host combines them.  If the structures exceed the LDS budget the
 // kernel only raises kFlagFallback.
+//
+// What bounds it is latency: a chain of barriers, LDS round trips and
+// cross-lane steps, most of it the same in every workgroup.  So combinations
+// over a wave are DPP scans, the bits of a narrow C span are spread over the
+// block's threads, words away from the slice are summed without a walk over
+// their bits, only the words in use are cleared, and no barrier waits for the
+// stores at the end.  Whole plan call (launch, kernel, the copy back), before
+// and after these: 21 x 21 full bands 28.5 -> 23.1 us, 121 x 121 39.0 ->
+// 28.5, 301 x 301 89 -> 45, 7 x 7 stencil 28.7 -> 25.9, 300 x 300 random
+// offsets within 30000 128 -> 115.
 // ---------------------------------------------------------------------------
-
-template <typename T, typename Op>
-__device__ __forceinline__ T wave_reduce(T v, Op op)
-{
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) v = op(v, __shfl_xor(v, s, 64));
-    return v;
-}
 
 // Combination of the kFastWaves per-wave values in slot[] (after a barrier).
 template <typename T, typename Op>
@@ -476,6 +479,7 @@ __device__ int64_t fast_select(const uint32_t* bits, const int32_t* pfx, int32_t
 
 __device__ __forceinline__ int32_t i32min(int32_t x, int32_t y) { return x < y ? x : y; }
 __device__ __forceinline__ int32_t i32max(int32_t x, int32_t y) { return x > y ? x : y; }
+__device__ __forceinline__ int32_t i32add(int32_t x, int32_t y) { return x + y; }
 __device__ __forceinline__ int32_t i32or(int32_t x, int32_t y) { return x | y; }
 __device__ __forceinline__ int64_t i64add(int64_t x, int64_t y) { return x + y; }
 __device__ __forceinline__ int64_t i64max(int64_t x, int64_t y) { return x > y ? x : y; }
@@ -497,12 +501,12 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
     int32_t* __restrict__ wg_max, int32_t* __restrict__ records, int32_t* __restrict__ wg_rec)
 {
     extern __shared__ uint32_t lds[];
-    __shared__ int32_t s32[8][kFastWaves];        // one slot per combined value
+    __shared__ int32_t s32[7][kFastWaves];        // one slot per combined value
     __shared__ int64_t s64[10][kFastWaves];
     __shared__ int32_t sscan[3][kFastWaves];
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int G = (int)gridDim.x, wg = (int)blockIdx.x;
-    const bool lane0 = lane == 0;
+    const bool lane0 = lane == 0, lane63 = lane == 63;   // 63 holds a wave's combination
 
     // LDS: the operand tables, then the bitmaps and this slice's C offsets
     int64_t* ast = reinterpret_cast<int64_t*>(lds);
@@ -516,7 +520,7 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
     const int64_t free_words = kFastLdsWords - fast_table_words(na, nb);
 
     // 1. operand tables into LDS; validity, ranges, value extents.  The
-    //    bitmap area is cleared meanwhile (whatever part the spans use).
+    //    first kFastClear words of the bitmap area are cleared meanwhile.
     int32_t amin = INT_MAX, amax = INT_MIN, bmin = INT_MAX, bmax = INT_MIN, bad = 0;
     int64_t aext = 0, bext = 0;
     for (int a = tid; a < na; a += kFastBlock) {
@@ -547,22 +551,16 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
             bext = i64max(bext, s0 + l);
         }
     }
-    {   // bitbase is 16-byte aligned when the tables are (5 na + 4 nb words)
-        const int64_t lead = (4 - (fast_table_words(na, nb) & 3)) & 3;
-        for (int64_t w = tid; w < lead && w < free_words; w += kFastBlock) bitbase[w] = 0u;
-        uint4* q = reinterpret_cast<uint4*>(bitbase + lead);
-        const int64_t nq = (free_words - lead) >> 2;
-        for (int64_t w = tid; w < nq; w += kFastBlock) q[w] = uint4{0u, 0u, 0u, 0u};
-        for (int64_t w = lead + 4 * nq + tid; w < free_words; w += kFastBlock) bitbase[w] = 0u;
-    }
-    bad = wave_reduce(bad, i32or);
-    amin = wave_reduce(amin, i32min);
-    amax = wave_reduce(amax, i32max);
-    bmin = wave_reduce(bmin, i32min);
-    bmax = wave_reduce(bmax, i32max);
-    aext = wave_reduce(aext, i64max);
-    bext = wave_reduce(bext, i64max);
-    if (lane0) {
+    const int64_t cleared = free_words < kFastClear ? free_words : kFastClear;
+    for (int64_t w = tid; w < cleared; w += kFastBlock) bitbase[w] = 0u;
+    bad = wave_scan_dpp(bad, 0, i32or);
+    amin = wave_scan_dpp(amin, INT_MAX, i32min);
+    amax = wave_scan_dpp(amax, INT_MIN, i32max);
+    bmin = wave_scan_dpp(bmin, INT_MAX, i32min);
+    bmax = wave_scan_dpp(bmax, INT_MIN, i32max);
+    aext = wave_scan_dpp(aext, (int64_t)0, i64max);   // extents are >= 0
+    bext = wave_scan_dpp(bext, (int64_t)0, i64max);
+    if (lane63) {
         s32[0][wave] = bad;
         s32[1][wave] = amin;
         s32[2][wave] = amax;
@@ -630,6 +628,10 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
     uint32_t* cbits = reinterpret_cast<uint32_t*>(bpfx + wb);
     int32_t* cpfx = reinterpret_cast<int32_t*>(cbits + wc);
     int32_t* rows = cpfx + wc;                       // the slice's C offsets
+    if (2 * (wa + wb + wc) > cleared) {
+        for (int64_t w = cleared + tid; w < 2 * (wa + wb + wc); w += kFastBlock) bitbase[w] = 0u;
+        __syncthreads();
+    }
 
     // a bit already set is a repeated offset; distinct offsets lo + index are
     // a contiguous band in order
@@ -646,9 +648,37 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
         const uint32_t m = 1u << (q & 31);
         if (atomicOr(&bbits[q >> 5], m) & m) dup |= kFlagBDup;
     }
+    // C's presence bits.  Where B's offsets are dense in their span, B's
+    // words are ORed in shifted by each A offset: na (wb + 1) word updates
+    // spread over the C span instead of na nb single-bit ones, of which up
+    // to 32 lanes at a time hit one word.  Whole plan call, bits against
+    // words: 61 x 61 full bands 24.8 / 24.0 us, 121 x 121 33.9 / 28.5; up to
+    // 45 x 45 the two are level (the words need one more barrier), and
+    // scattered offsets (words mostly empty) have few bits in one word.
+    const bool by_words = 4 * (wb + 1) <= nb && (int64_t)na * nb >= 2048;
+    if (by_words) {
+        __syncthreads();
+        const uint32_t top = (SC & 31) ? (1u << (SC & 31)) - 1u : 0xffffffffu;
+        const int32_t nw = (int32_t)wb, items = na * nw;
+        for (int32_t t = tid; t < items; t += kFastBlock) {
+            const int32_t a = t / nw, w = t - a * nw;
+            // position of this B word's bit 0 in the C span: negative where
+            // the span's low end is cut at 1 - n
+            const int64_t q = (int64_t)aoff[a] + bmin - clo + 32 * (int64_t)w;
+            const uint64_t v = (uint64_t)bbits[w] << (q & 31);
+            const int64_t c = q >> 5;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                uint32_t x = (uint32_t)(v >> (32 * j));
+                if (c + j == wc - 1) x &= top;
+                if (x && c + j >= 0 && c + j < wc) atomicOr(&cbits[c + j], x);
+            }
+        }
+    }
     // sums: lanes over B (offsets held in registers, 4 per lane at a time),
     // waves over A; pair count, useful flops
-    int64_t np = 0, fl = 0;
+    int32_t mine_np = 0;                             // na nb <= kFastMaxProducts
+    int64_t fl = 0;
     for (int b0 = 0; b0 < nb; b0 += 4 * 64) {
         int db[4];
         bool has[4];
@@ -672,8 +702,8 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
                     const int64_t dc = (int64_t)da + db[j];
                     if (has[j] && dc > -(int64_t)n && dc < n) {
                         const int64_t q = dc - clo;
-                        atomicOr(&cbits[q >> 5], 1u << (q & 31));
-                        ++np;
+                        if (!by_words) atomicOr(&cbits[q >> 5], 1u << (q & 31));
+                        ++mine_np;
                         int m = iabs_(da) > iabs_(db[j]) ? iabs_(da) : iabs_(db[j]);
                         m = iabs_((int)dc) > m ? iabs_((int)dc) : m;
                         fl += 2 * (int64_t)(n - m);
@@ -682,17 +712,17 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
             }
         }
     }
-    dup = wave_reduce(dup, i32or);
-    np = wave_reduce(np, i64add);
-    fl = wave_reduce(fl, i64add);
-    if (lane0) {
+    dup = wave_scan_dpp(dup, 0, i32or);
+    mine_np = wave_scan_dpp(mine_np, 0, i32add);
+    fl = wave_scan_dpp(fl, (int64_t)0, i64add);
+    if (lane63) {
         s32[5][wave] = dup;
-        s64[2][wave] = np;
+        s64[2][wave] = mine_np;
         s64[3][wave] = fl;
     }
     __syncthreads();                                                   // barrier 2
     dup = combine_waves(s32[5], i32or);
-    np = combine_waves(s64[2], i64add);
+    const int64_t np = combine_waves(s64[2], i64add);
     fl = combine_waves(s64[3], i64add);
     const int32_t contiguous = (dup & kNotContiguous) ? 0 : 1;
     dup &= ~kNotContiguous;
@@ -721,8 +751,8 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
                 t += (w0 + i < nw[j]) ? __popc(bm[j][w0 + i]) : 0;
             }
             tot[j] = t;
-            incl[j] = wave_inclusive_scan(t);
-            if (lane == 63) sscan[j][wave] = incl[j];
+            incl[j] = wave_scan_dpp(t, 0, i32add);
+            if (lane63) sscan[j][wave] = incl[j];
         }
         __syncthreads();
         int32_t before[3] = {0, 0, 0}, sum[3] = {0, 0, 0};
@@ -755,20 +785,44 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
         return fast_rank(bbits, bpfx, x - bmin);
     };
     const int64_t k0 = nC * wg / G, k1 = nC * (wg + 1) / G;
+    // 2^sub threads per word while the block covers all words at once (a
+    // thread's bits are walked one after the other): a narrow C span is done
+    // in one step instead of up to 32
+    int sub = 0;
+    while (sub < 5 && (wc << (sub + 1)) <= kFastBlock) ++sub;
+    const int width = 32 >> sub;
     int64_t lb = 0, nz = 0;
-    for (int64_t w = tid; w < wc; w += kFastBlock) {
-        int64_t r = cpfx[w];
-        for (uint32_t m = cbits[w]; m; m &= m - 1u, ++r) {
-            const int64_t o = clo + w * 32 + (__ffs(m) - 1);
-            const int64_t len = (int64_t)n - (o < 0 ? -o : o);
+    for (int64_t t = tid; t < (wc << sub); t += kFastBlock) {
+        const int64_t w = t >> sub;
+        const uint32_t all = cbits[w];
+        const int at = (int)(t & ((1 << sub) - 1)) * width;      // this thread's lowest bit
+        uint32_t m = all & ((0xffffffffu >> (32 - width)) << at);
+        if (!m) continue;
+        int32_t r = cpfx[w] + __popc(all & ((1u << at) - 1u));
+        const int32_t p = __popc(m), o0 = (int32_t)(clo + w * 32);
+        // all below or all above the slice, and of one sign: the sums of the
+        // offsets come from the bit positions' binary digits, without a walk
+        if ((r + p <= k0 || r >= k1) && (o0 >= 0 || o0 + 31 <= 0)) {
+            const int32_t digits = __popc(m & 0xaaaaaaaau) + 2 * __popc(m & 0xccccccccu) +
+                                   4 * __popc(m & 0xf0f0f0f0u) + 8 * __popc(m & 0xff00ff00u) +
+                                   16 * __popc(m & 0xffff0000u);
+            const int64_t sum = (int64_t)p * o0 + digits;
+            const int64_t len = (int64_t)p * n - (o0 >= 0 ? sum : -sum);
             nz += len;
             lb += r < k0 ? len : 0;
-            if (r >= k0 && r < k1) rows[r - k0] = (int32_t)o;
+            continue;
+        }
+        for (; m; m &= m - 1u, ++r) {
+            const int32_t o = o0 + (__ffs(m) - 1);
+            const int32_t len = n - iabs_(o);
+            nz += len;
+            lb += r < k0 ? len : 0;
+            if (r >= k0 && r < k1) rows[r - k0] = o;
         }
     }
-    lb = wave_reduce(lb, i64add);
-    nz = wave_reduce(nz, i64add);
-    if (lane0) {
+    lb = wave_scan_dpp(lb, (int64_t)0, i64add);
+    nz = wave_scan_dpp(nz, (int64_t)0, i64add);
+    if (lane63) {
         s64[5][wave] = lb;
         s64[6][wave] = nz;
     }
@@ -780,8 +834,8 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
         int64_t pb = 0;
         for (int a = tid; a < na; a += kFastBlock)
             pb += rank_b(d0 - aoff[a]) - rank_b(1 - (int64_t)n - aoff[a]);
-        pb = wave_reduce(pb, i64add);
-        if (lane0) s64[4][wave] = pb;
+        pb = wave_scan_dpp(pb, (int64_t)0, i64add);
+        if (lane63) s64[4][wave] = pb;
         lbase = combine_waves(s64[5], i64add);
     }
     int32_t flags = 0;
@@ -791,6 +845,10 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
     if (flags) return;
     if (records && wg == 0 && tid == 0)   // the 4 ints after the records
         reinterpret_cast<int4*>(records)[np] = int4{0, 0, amin, amax};
+    // the workgroup's flag word: zeroed here, before barrier 4, and set after
+    // it by a wave that finds a flag (a reduction at the end would hold all
+    // waves at a barrier until their stores have drained)
+    if (records && tid == 0) wg_rec[wg] = 0;
 
     // 4. each wave's run of C diagonals: counts, then one exchange
     const int64_t R = k1 - k0;
@@ -879,12 +937,7 @@ __global__ __launch_bounds__(kFastBlock) void k_sym_fast(
             slot += __popcll(m);
         }
     }
-    if (records) {   // one word per workgroup: the host ORs them
-        rflag = wave_reduce(rflag, i32or);
-        if (lane0) s32[7][wave] = rflag;
-        __syncthreads();
-        if (tid == 0) wg_rec[wg] = combine_waves(s32[7], i32or);
-    }
+    if (records && __any(rflag) && lane0) wg_rec[wg] = 1;   // the host ORs the words
 
     // 6. lookup: every offset of the 2n - 1, grid-stride over all workgroups
     if (lookup) {

@@ -392,6 +392,28 @@ def test_band_kernel_same_bits_as_gather(dev, oracle, n, offs_a, offs_b):
         check_values(Cb.cpu().numpy(), want, ab)
 
 
+# B dense in its span from 2048 products on (its bitmap's words are ORed into
+# C's): bands cut at both ends of (-n, n), a C span that fills its last word,
+# gaps, reversed operands; one product fewer than the rule asks for; spans
+# beyond the words cleared up front, whose words are summed without a walk.
+SYM_SHAPES = [
+    (70, range(-69, 70), range(-69, 70)), (4096, range(-32, 32), range(-32, 33)),
+    (300, range(299, 100, -1), range(250, 299)), (300, range(-299, -230), range(-299, -200)),
+    (5000, range(-4999, 5000, 157), range(-40, 41)), (999, range(0, 16), range(-64, 64)),
+    (999, range(0, 16), range(-64, 63)), (2000, range(-90, 91, 3), [-900, *range(800, 1999)]),
+    (40000, range(-39999, 40000, 1601), range(-9000, 9001, 1007)),
+    (1 << 20, range(-50000, 50001, 2003), [-49999, -31, -1, 0, 1, 33, 50001]),
+]
+
+
+@pytest.mark.parametrize("n,oa,ob", SYM_SHAPES, ids=range(len(SYM_SHAPES)))
+def test_symbolic_bitmaps(dev, oracle, n, oa, ob):
+    A = workloads.hm_random(n, list(oa), 1, dev)
+    B = workloads.hm_random(n, list(ob), 2, dev)
+    check_plan(oracle, SpgemmPlan(A, B, want_lookup=n < 10000), A, B)
+    check_plan(oracle, SpgemmPlan(B, A), B, A)
+
+
 def test_band_kernel_choice_and_capacity(dev):
     """auto picks the band kernel for gemm_diag's contiguous bands from 1024
     row blocks on (the A-stationary kernel below that) and the gather for
