@@ -24,7 +24,7 @@ template <int Ctrl, int RowMask> __device__ __forceinline__ double dpp_add(doubl
 }
 
 // The wave's sum, in lane 63: within rows of 16 lanes, then across the rows
-// (a sixth of the latency of six cross-lane permutes).
+// (moves between registers, no round trip through LDS hardware per step).
 __device__ __forceinline__ double wave_sum63(double x)
 {
     x = dpp_add<0x111, 0xf>(x);   // row_shr:1

@@ -412,7 +412,8 @@ __device__ __forceinline__ void straight_chunk(int64_t r, int64_t cols, int m,
 // Few rows, many diagonals (split_waves): S waves share one tile of 64 R
 // rows, wave w accumulating the diagonals [K w / S, K (w + 1) / S), and the
 // S sums of each row are added in wave order through LDS (a fixed order:
-// deterministic).
+// deterministic).  The shorter sums round less: fp64, n = 100003, K = 64
+// against an 80-bit sum 2.7e-16 in one sum, 1.45e-16 in eight.
 //
 // What bounds such a call is the chain of load latencies of one wave over
 // its K diagonals, with too few waves to hide it (fp64, n = 100003, K = 64:
