@@ -437,9 +437,10 @@ void launch_resident(const Resident& p, int32_t n, int32_t K, const int32_t* off
 // launch between them.  For rows above the resident range: n = 360000 401 ->
 // 346 us, level with the three launches at 600000 (m = 30), and slower above,
 // where the columns' 16 runs a lane through the vector L1 cost more than the
-// launches (n = 2^22: 63 us a step against 53); so it ends at kFusedRows.  The grid is at most kFusedWgs workgroups, each over
-// tiles of 512 rows of its XCD's range in step with the others, so that the
-// next launch can add all parts at its start in every workgroup.
+// launches (n = 2^22: 63 us a step against 53); so it ends at kFusedRows.
+// The grid is at most kFusedWgs workgroups, each over tiles of 512 rows of its
+// XCD's range in step with the others, so that the next launch can add all
+// parts at its start in every workgroup.
 // ---------------------------------------------------------------------------
 constexpr int kFusedMax = 7;
 constexpr int kFusedRows = 500000;
@@ -689,9 +690,10 @@ Layout layout(int64_t n, int m)
     const bool small = n <= 2 * 512 * (int64_t)kMaxResident;
     if (small) off += align256((size_t)(m + 1) * kMaxResident * kPart * sizeof(double));
     L.zbuf = off;   // four z of a resident launch, two of the fused steps
-    off += align256((small ? 4 : 2) * (size_t)n * sizeof(cf32));
+    const bool fused = n <= kFusedRows;   // every resident size lies below
+    if (fused) off += align256((small ? 4 : 2) * (size_t)n * sizeof(cf32));
     L.parts = off;
-    off += align256(4 * kFusedWgs * sizeof(double));
+    if (fused) off += align256(4 * kFusedWgs * sizeof(double));
     L.total = off;
     return L;
 }
