@@ -800,15 +800,23 @@ int launch_astat(const char* fn, int32_t n, const int32_t* A_off, const int64_t*
             rounds_ok(16, astat_slots<T, 16>(nA)))
             return DIAGPU_ASTAT_LAUNCH(16);
         // many C diagonals: 8, where two workgroups still fit a CU, from 4
-        // rounds, or from n = 100000 where the C diagonals average 3 entries
+        // rounds, or for a narrow A (a stencil) from n = 150000 where the C
+        // diagonals average 3 entries and the blocks don't just miss a round
         // (us, 4 rows -> 8: the 7-point stencil times its 63, 129 and 231
         // diagonals at n = 604800 113 -> 90, 303 -> 277, 557 -> 482, at 409600
         // 78 -> 67, 152 -> 138, 371 -> 337, at 151951 30 -> 28, 51.4 -> 51.1,
-        // 102 -> 89, at 27000 7.9 -> 8.1, 11.3 -> 11.7; plans of about one
+        // 102 -> 89; 7 x 60 neighbouring offsets at 100000 14.0 -> 15.4, 200000
+        // 28.6 -> 26.3, 10^6 145 -> 121; 7 x 140 at 300000, 1.1 rounds, 0.99 of
+        // the rate.  More A diagonals lose as often as they gain below 4
+        // rounds: 33 x 60 at 100000 38 -> 43, 200000 74 -> 71, 300000 0.86 of
+        // the rate, 400000 129 -> 138, 10^6 390 -> 370.  Plans of about one
         // entry per C diagonal lose: 5 x 120 at n = 150000 71 -> 79, 400000 177
         // -> 224)
+        const int64_t blocks8 = ceil_div<int64_t>(n, 512), slots8 = astat_slots<T, 8>(nA);
+        const bool just_over = blocks8 > slots8 && 4 * blocks8 < 5 * slots8;
         if (c_ndiag > 4 * kWaves && nA <= Astat<T, 8>::kMax2 &&
-            (rounds_ok(8, astat_slots<T, 8>(nA)) || (n >= 100000 && n_pairs >= 3 * c_ndiag)))
+            (rounds_ok(8, slots8) ||
+             (nA <= 8 && n >= 150000 && n_pairs >= 3 * c_ndiag && !just_over)))
             return DIAGPU_ASTAT_LAUNCH(8);
     } else if constexpr (kForceR == 0) {
         // complex: 8 where every wave has at most one C diagonal

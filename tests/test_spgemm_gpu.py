@@ -1015,14 +1015,14 @@ def test_full_only_for_contiguous_bands_in_order(dev):
                        plan.multiply(A.values, A.values, kernel="gather"))
 
 
-# Launch shapes of the A-stationary kernel: 8 rows per lane from n = 100000 for
-# plans of at least 3 entries per C diagonal, complex values split over two
+# Launch shapes of the A-stationary kernel: 8 rows per lane from n = 150000 for
+# a narrow A and plans of at least 3 entries per C diagonal, complex values split over two
 # workgroups per block from 100 C diagonals, and XCDs interleaved in runs of 4
 # blocks where C holds 225 million values (1000003 rows: the last run partly
 # empty).  The operand S is the stencil's power S = (I + H)^k on an nx x ny
 # plane, k steps wide.  Bits of the gather.
 @pytest.mark.parametrize("n,nx,ny,k,dtype", [
-    (99999, 40, 50, 3, torch.float32), (100000, 40, 50, 3, torch.float32),
+    (149999, 40, 50, 3, torch.float32), (150000, 40, 50, 3, torch.float32),
     (150001, 33, 77, 4, torch.float32), (12345, 17, 23, 3, torch.complex64),
     (70001, 33, 47, 3, torch.complex64), (200003, 33, 47, 3, torch.complex64),
     (1000003, 101, 99, 4, torch.float32)])
