@@ -21,9 +21,10 @@
 // not needed before step j+1's update, so its sum shares one launch with
 // step j+1's d sum (sum_partials2): three launches per step.
 //
-// These are three launches a step for large n; small n and few diagonals run
-// all steps in one launch (k_lanczos_resident), and sizes between in one
-// launch a step (k_lanczos_step), with the same recurrence.
+// These are three launches a step for large n or many diagonals; few diagonals
+// up to kFusedRows rows run in one launch a step (k_lanczos_step), with the
+// same recurrence.  Which of the two is a rule on n, K and the workspace alone,
+// so equal calls give equal bits whatever else runs on the device.
 //
 // After m steps the host reads alpha and beta (the only synchronisation, one
 // copy), forms T_m = tridiag(beta, alpha, beta) and evaluates
@@ -35,8 +36,6 @@
 // ||psi_0|| beta_m |c_m| is returned.
 #include <cmath>
 #include <complex>
-#include <cstring>
-#include <mutex>
 #include <type_traits>
 #include <vector>
 
@@ -146,69 +145,6 @@ __global__ __launch_bounds__(kVB) void k_lanczos_update(cf32* __restrict__ zw,
     store_partial<kVB>(s, tile, partials);
 }
 
-// ---------------------------------------------------------------------------
-// Lanczos steps in one launch, for an H of at most 9 diagonals and rows that
-// fit the chip's registers (resident_rows).  At these sizes a step of three
-// launches takes 11.5 us whatever it moves (m = 30: 345 to 380 us a call up to
-// n = 262144).  What bounds a step here is one exchange between all
-// workgroups: 2.0 us for 4 workgroups, 3.3 for 78, 5.8 at n = 262144, where
-// the columns' z count too.  Calls with m = 30 (5 diagonals): n = 1024 353 ->
-// 104 us, 19881 353 -> 136, 65536 356 -> 152, 262144 378 -> 219.
-//
-// Lane rows: workgroup b owns RL BS consecutive rows, RL per lane.  A lane
-// keeps H's values for its rows, its own u_j and u_{j-1}, and u_j and u_{j-1}
-// at the K columns its rows read -- the same values the owning lanes hold,
-// since every lane forms u_{j+1} from z_j by the same operations.  So a step
-// exchanges only z_j and the sums d_j and q_{j-1}:
-//   z_j = H u_j, stored to zbuf[j mod 4]; the workgroup's parts of d_j and
-//   q_{j-1} = ||u_j||^2 stored to slot j; every workgroup reads all parts of
-//   slot j, waiting for each, and adds them in one order; u_{j+1} at its rows
-//   and columns from z_j, waiting for each z_j it reads.
-// Every value waits for itself: a slot or a zbuf element holds kUnset (a NaN
-// that no arithmetic on H and psi makes) until it is written, so nothing is
-// ordered against anything else and no release fence is needed (it would
-// write back the XCD's L2 each step).  All exchanged values are agent-scope
-// relaxed atomics of 8 bytes, coherent between the XCDs.  Slots are written
-// once, after a launch before this one has set them to kUnset (zbuf too).  At
-// step j a lane sets its rows of zbuf[(j + 2) mod 4], which hold z_{j-2}, back
-// to kUnset: it has every workgroup's parts of j - 1, each stored after that
-// workgroup had read all its z_{j-2}; and the lane's wave waits for its own
-// z_j loads, issued after that store (vector memory operations of a wave
-// complete in order), before its workgroup stores its parts of j + 1, which
-// every workgroup has before it reads zbuf[(j + 2) mod 4] for z_{j+2}.
-//
-// The workgroups wait for each other, so all of them have to be on the chip
-// at once: at most one per CU, one such launch at a time in a process
-// (resident_lock), and a wait that ends after kWaitTicks in any case, after
-// which q[m] is left at kUnset and the host takes the launches per step.
-// ---------------------------------------------------------------------------
-constexpr uint64_t kUnset = 0x7FF8C0DEC0DEC0DFull;
-constexpr uint64_t kWaitTicks = 100000000ull;   // of the 100 MHz clock: 1 s
-constexpr int kMaxResident = 256;               // workgroups (one lane polls one)
-// 64-bit words of a workgroup's parts of a step: two values, alone in 64 bytes
-// (packed, the polls and stores of eight workgroups share a line: 3.9 against
-// 3.3 us a step with 78 workgroups).
-constexpr int kPart = 8;
-
-inline __device__ void share(uint64_t* p, uint64_t v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-inline __device__ uint64_t shared_value(const uint64_t* p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__global__ __launch_bounds__(256) void k_unset(uint64_t* __restrict__ slots, int count,
-                                              uint64_t* __restrict__ zbuf, int zcount,
-                                              uint64_t* __restrict__ last)
-{
-    const int i0 = (int)(blockIdx.x * 256 + threadIdx.x), step = (int)(gridDim.x * 256);
-    if (i0 == 0) *last = kUnset;
-    for (int i = i0; i < count; i += step) slots[i] = kUnset;
-    for (int i = i0; i < zcount; i += step) zbuf[i] = kUnset;
-}
-
 // Both sums over the workgroup, in every lane; a fixed order.
 template <int BS> __device__ __forceinline__ void block_sum2(double& a, double& b, double (*ws)[2])
 {
@@ -228,205 +164,6 @@ template <int BS> __device__ __forceinline__ void block_sum2(double& a, double& 
     }
 }
 
-// slots: [m + 1][gridDim.x][kPart]; zbuf: [4][n]; rest: u_2, u_3, ... n
-// apart.  K <= KM.
-template <typename TV, int KM, int RL, int BS>
-__global__ __launch_bounds__(BS) void k_lanczos_resident(
-    int32_t n, int32_t K, const int32_t* __restrict__ offs, const TV* __restrict__ vals,
-    const cf32* __restrict__ psi0, int m, cf32* __restrict__ rest, uint64_t* zbuf,
-    uint64_t* slots, double* __restrict__ d_out, double* __restrict__ q_out)
-{
-    __shared__ double ws[4][BS / 64][2];   // two sums a step, two steps in turn
-    __shared__ int dead;                   // a wait for z given up: no more parts
-    if (threadIdx.x == 0) dead = 0;        // (a barrier follows before its first use)
-    const int wg = (int)blockIdx.x, G = (int)gridDim.x, tid = (int)threadIdx.x;
-    TV h[RL][KM];
-    cf32 u[RL][KM], up[RL][KM], uo[RL], upo[RL];
-    int col[RL][KM];
-    uint32_t ok[RL];
-#pragma unroll
-    for (int r = 0; r < RL; ++r) {
-        const int row = (wg * RL + r) * BS + tid;
-        const bool in = row < n;
-        uo[r] = in ? psi0[row] : cf32{0.f, 0.f};
-        upo[r] = cf32{0.f, 0.f};
-        ok[r] = 0;
-#pragma unroll
-        for (int k = 0; k < KM; ++k) {
-            const int64_t c = (int64_t)row + (k < K ? offs[k] : 0);
-            const bool has = in && k < K && c >= 0 && c < n;
-            ok[r] |= has ? 1u << k : 0u;
-            col[r][k] = has ? (int)c : 0;
-            h[r][k] = has ? vals[(int64_t)k * n + c] : zero_of<TV>();
-            u[r][k] = psi0[col[r][k]];
-            up[r][k] = cf32{0.f, 0.f};
-        }
-    }
-    // waits for every workgroup's parts of a step; false: given up
-    auto gather = [&](const uint64_t* at, double& a, double& b) -> bool {
-        uint64_t x = 0, y = 0;
-        bool gave_up = false;
-        if (tid < G) {
-            const uint64_t began = __builtin_amdgcn_s_memrealtime();
-            for (;;) {
-                x = shared_value(at + kPart * tid);
-                y = shared_value(at + kPart * tid + 1);
-                if (x != kUnset && y != kUnset) break;
-                if (__builtin_amdgcn_s_memrealtime() - began > kWaitTicks) {
-                    gave_up = true;
-                    break;
-                }
-            }
-        }
-        a = __builtin_bit_cast(double, x);
-        b = __builtin_bit_cast(double, y);
-        return __syncthreads_or(gave_up) == 0;
-    };
-    double s_prev = 0.0, q_prev = 0.0;
-    for (int j = 1; j <= m; ++j) {
-        uint64_t* zb = zbuf + (int64_t)(j & 3) * n;
-        uint64_t* clear = zbuf + (int64_t)((j + 2) & 3) * n;   // holds z_{j-2}
-        cf32 z[RL];
-        double d = 0.0, q = 0.0;
-#pragma unroll
-        for (int r = 0; r < RL; ++r) {
-            z[r] = cf32{0.f, 0.f};
-#pragma unroll
-            for (int k = 0; k < KM; ++k)
-                z[r] = sel((ok[r] >> k) & 1u, mad(z[r], h[r][k], u[r][k]), z[r]);
-            const int row = (wg * RL + r) * BS + tid;
-            if (row < n) {
-                share(zb + row, __builtin_bit_cast(uint64_t, z[r]));
-                share(clear + row, kUnset);
-            }
-            d += dotpart(uo[r], z[r]);
-            q += dotpart(uo[r], uo[r]);
-        }
-        block_sum2<BS>(d, q, ws[2 * (j & 1)]);
-        uint64_t* at = slots + (int64_t)(j - 1) * G * kPart;
-        if (tid == 0 && !dead) {
-            share(at + kPart * wg, __builtin_bit_cast(uint64_t, d));
-            share(at + kPart * wg + 1, __builtin_bit_cast(uint64_t, q));
-        }
-        // z_j at the columns, asked for ahead of the wait for the parts (one
-        // row per lane: more would not fit the registers); what has not come
-        // by then is asked for again below
-        uint64_t zc[RL][KM];
-        if constexpr (RL == 1)
-#pragma unroll
-            for (int k = 0; k < KM; ++k) zc[0][k] = shared_value(zb + col[0][k]);
-        if (!gather(at, d, q)) return;   // q_out[m] stays unset
-        if constexpr (RL > 1)
-#pragma unroll
-            for (int r = 0; r < RL; ++r)
-#pragma unroll
-                for (int k = 0; k < KM; ++k) zc[r][k] = shared_value(zb + col[r][k]);
-        block_sum2<BS>(d, q, ws[2 * (j & 1) + 1]);
-        if (wg == 0 && tid == 0) {
-            d_out[j - 1] = d;
-            q_out[j - 1] = q;
-        }
-        // the scalars of k_lanczos_update
-        const double sj = sqrt(q);
-        const float inv_s = q > 0.0 ? (float)(1.0 / sj) : 0.f;
-        const float alpha = q > 0.0 ? (float)(d / q) : 0.f;
-        const float ratio = j >= 2 && q_prev > 0.0 ? (float)(sj / s_prev) : 0.f;
-        s_prev = sj;
-        q_prev = q;
-        auto next = [&](const cf32& zv, cf32& uc, cf32& pc) {
-            float re = __builtin_fmaf(-alpha, uc.re, zv.re) * inv_s;
-            float im = __builtin_fmaf(-alpha, uc.im, zv.im) * inv_s;
-            if (j >= 2) {
-                re = __builtin_fmaf(-ratio, pc.re, re);
-                im = __builtin_fmaf(-ratio, pc.im, im);
-            }
-            pc = uc;
-            uc = cf32{re, im};
-        };
-        const uint64_t began = __builtin_amdgcn_s_memrealtime();
-        bool gave_up = false;
-#pragma unroll
-        for (int r = 0; r < RL; ++r)
-#pragma unroll
-            for (int k = 0; k < KM; ++k)
-                while (((ok[r] >> k) & 1u) && zc[r][k] == kUnset && !gave_up) {
-                    zc[r][k] = shared_value(zb + col[r][k]);
-                    gave_up = __builtin_amdgcn_s_memrealtime() - began > kWaitTicks;
-                }
-        if (gave_up) dead = 1;
-#pragma unroll
-        for (int r = 0; r < RL; ++r) {
-            next(z[r], uo[r], upo[r]);
-            const int row = (wg * RL + r) * BS + tid;
-            if (j < m && row < n) rest[(int64_t)(j - 1) * n + row] = uo[r];
-#pragma unroll
-            for (int k = 0; k < KM; ++k) next(__builtin_bit_cast(cf32, zc[r][k]), u[r][k], up[r][k]);
-        }
-    }
-    // q_m = ||u_{m+1}||^2: workgroup 0 adds the parts
-    double q = 0.0, unused = 0.0;
-#pragma unroll
-    for (int r = 0; r < RL; ++r) q += dotpart(uo[r], uo[r]);
-    block_sum2<BS>(q, unused, ws[2 * ((m + 1) & 1)]);
-    uint64_t* at = slots + (int64_t)m * G * kPart;
-    if (tid == 0 && !dead) {
-        share(at + kPart * wg, __builtin_bit_cast(uint64_t, q));
-        share(at + kPart * wg + 1, __builtin_bit_cast(uint64_t, q));
-    }
-    if (wg != 0 || !gather(at, q, unused)) return;
-    block_sum2<BS>(q, unused, ws[2 * ((m + 1) & 1) + 1]);
-    if (tid == 0) q_out[m] = q;
-}
-
-// Threads per workgroup and rows per lane of a resident launch; 0 rows: not
-// taken.  At most one workgroup per CU, whose lanes then have 256 registers
-// each: 2 rows of up to 9 diagonals (four rows spilled, and lost to the fused
-// steps).  512 threads rather than 256 or 1024: fewer workgroups to wait for
-// against more waves in each of them (n = 65536: 3.8 us a step, 4.7 and 5.1);
-// 256 where that leaves a few workgroups (n = 1024: 2.0 against 2.2).
-struct Resident {
-    int rows_per_lane, threads, wgs;
-};
-
-Resident resident_rows(int32_t n, int32_t K, int cus)
-{
-    const int most = cus < kMaxResident ? cus : kMaxResident;
-    Resident p{0, 0, 0};
-    if (K < 1 || K > 9) return p;
-    p.threads = n <= 16384 ? 256 : 512;
-    const int64_t per = (int64_t)p.threads * most;
-    p.rows_per_lane = n <= per ? 1 : (n <= 2 * per ? 2 : 0);
-    if (p.rows_per_lane)
-        p.wgs = (int)((n + (int64_t)p.threads * p.rows_per_lane - 1) / (p.threads * p.rows_per_lane));
-    return p;
-}
-
-// One resident launch at a time in this process: a second caller takes the
-// launches per step meanwhile.
-std::mutex& resident_lock()
-{
-    static std::mutex mu;
-    return mu;
-}
-
-template <typename TV, int KM>
-void launch_resident(const Resident& p, int32_t n, int32_t K, const int32_t* offs, const TV* vals,
-                     const cf32* psi0, int m, cf32* rest, uint64_t* zbuf, uint64_t* slots, double* d,
-                     double* q, hipStream_t s)
-{
-#define DIAGPU_RESIDENT(RL, BS)                                                                  \
-    hipLaunchKernelGGL((k_lanczos_resident<TV, KM, RL, BS>), dim3((unsigned)p.wgs), dim3(BS), 0, s, \
-                       n, K, offs, vals, psi0, m, rest, zbuf, slots, d, q)
-    if (p.threads == 256) {
-        DIAGPU_RESIDENT(1, 256);
-    } else if (p.rows_per_lane == 1) {
-        DIAGPU_RESIDENT(1, 512);
-    } else {
-        DIAGPU_RESIDENT(2, 512);
-    }
-#undef DIAGPU_RESIDENT
-}
-
 // ---------------------------------------------------------------------------
 // One launch per step, for an H of at most kFusedMax diagonals: step j forms
 // u_{j+1} from z_j at its rows and at the columns its rows read, and from it
@@ -434,8 +171,7 @@ void launch_resident(const Resident& p, int32_t n, int32_t K, const int32_t* off
 // an update and a sum launch per step it reads z_j, u_j and u_{j-1} once for
 // both (the columns' copies come from the caches) and writes u_{j+1} and
 // z_{j+1} once: 60 instead of 68 bytes of HBM traffic a row at K = 5, and no
-// launch between them.  For rows above the resident range: n = 360000 401 ->
-// 346 us, level with the three launches at 600000 (m = 30), and slower above,
+// launch between them.  n = 360000 401 -> 346 us, level with the three launches at 600000 (m = 30), and slower above,
 // where the columns' 16 runs a lane through the vector L1 cost more than the
 // launches (n = 2^22: 63 us a step against 53); so it ends at kFusedRows.
 // The grid is at most kFusedWgs workgroups, each over tiles of 512 rows of its
@@ -661,7 +397,7 @@ __global__ __launch_bounds__(kVB) void k_combine(const cf32* __restrict__ first,
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 struct Layout {
-    size_t vecs, pd, pq, d, q, slots, zbuf, parts, total;   // pd: SpMV dot partials, pq: norm partials
+    size_t vecs, pd, pq, d, q, zbuf, parts, total;   // pd: SpMV dot partials, pq: norm partials
 };
 
 Layout layout(int64_t n, int m)
@@ -684,14 +420,9 @@ Layout layout(int64_t n, int m)
     L.d = off;   // d[m] and q[m+1] back to back: one copy to the host
     L.q = off + (size_t)m * sizeof(double);
     off += align256((size_t)(2 * m + 1) * sizeof(double));
-    // a resident launch's exchange (any CU count, so that the size does not
-    // depend on the device)
-    L.slots = off;
-    const bool small = n <= 2 * 512 * (int64_t)kMaxResident;
-    if (small) off += align256((size_t)(m + 1) * kMaxResident * kPart * sizeof(double));
-    L.zbuf = off;   // four z of a resident launch, two of the fused steps
-    const bool fused = n <= kFusedRows;   // every resident size lies below
-    if (fused) off += align256((small ? 4 : 2) * (size_t)n * sizeof(cf32));
+    L.zbuf = off;   // two z of the fused steps
+    const bool fused = n <= kFusedRows;
+    if (fused) off += align256(2 * (size_t)n * sizeof(cf32));
     L.parts = off;
     if (fused) off += align256(4 * kFusedWgs * sizeof(double));
     L.total = off;
@@ -733,26 +464,25 @@ int expm_krylov(int32_t rows, int32_t cols, int32_t K, const int32_t* offs, cons
 
     const int stiles = spmv_tiles<TV, cf32>(rows);
 
-    // Every step's launches; d[0 .. m) and q[0 .. m] are queued when it returns.
-    auto launches_per_step = [&]() -> int {
-        if (K >= 1 && K <= kFusedMax && rows <= kFusedRows) {
-            cf32* zbuf = reinterpret_cast<cf32*>(ws + L.zbuf);
-            double* parts = reinterpret_cast<double*>(ws + L.parts);
-            auto go = [&](auto km) {
-                fused_steps<TV, decltype(km)::value>(rows, K, offs, vals, psi0, m, vecs, zbuf,
-                                                     parts, d, q, s);
-            };
-            if (K <= 3)
-                go(std::integral_constant<int, 3>{});
-            else if (K <= 5)
-                go(std::integral_constant<int, 5>{});
-            else
-                go(std::integral_constant<int, 7>{});
-            return check_launch(fn);
-        }
+    int st;
+    if (K >= 1 && K <= kFusedMax && rows <= kFusedRows) {
+        cf32* zbuf = reinterpret_cast<cf32*>(ws + L.zbuf);
+        double* parts = reinterpret_cast<double*>(ws + L.parts);
+        auto go = [&](auto km) {
+            fused_steps<TV, decltype(km)::value>(rows, K, offs, vals, psi0, m, vecs, zbuf, parts, d,
+                                                 q, s);
+        };
+        if (K <= 3)
+            go(std::integral_constant<int, 3>{});
+        else if (K <= 5)
+            go(std::integral_constant<int, 5>{});
+        else
+            go(std::integral_constant<int, 7>{});
+        st = check_launch(fn);
+    } else {
         // pq holds the partials of q[j-1] when step j starts (||psi_0||^2 for j = 1)
         hipLaunchKernelGGL(k_norm2, vgrid, dim3(kVB), 0, s, psi0, n, vtiles, vper, pq);
-        int st = check_launch(fn);
+        st = check_launch(fn);
         if (st) return st;
         for (int j = 1; j <= m; ++j) {
             const cf32* uj = j == 1 ? psi0 : slot(j);
@@ -766,29 +496,8 @@ int expm_krylov(int32_t rows, int32_t cols, int32_t K, const int32_t* offs, cons
             st = check_launch(fn);
             if (st) return st;
         }
-        return sum_partials(pq, vtiles, q + m, stream);
-    };
-    // The same in one launch where it fits.
-    auto resident = [&](const Resident& p) -> int {
-        uint64_t* slots = reinterpret_cast<uint64_t*>(ws + L.slots);
-        uint64_t* zbuf = reinterpret_cast<uint64_t*>(ws + L.zbuf);
-        const int count = kPart * (m + 1) * p.wgs;
-        hipLaunchKernelGGL(k_unset, dim3(rows < (1 << 16) ? 64 : 1024), dim3(256), 0, s, slots, count,
-                           zbuf, 4 * rows, reinterpret_cast<uint64_t*>(q + m));
-        if (K <= 3)
-            launch_resident<TV, 3>(p, rows, K, offs, vals, psi0, m, vecs, zbuf, slots, d, q, s);
-        else if (K <= 5)
-            launch_resident<TV, 5>(p, rows, K, offs, vals, psi0, m, vecs, zbuf, slots, d, q, s);
-        else if (K <= 7)
-            launch_resident<TV, 7>(p, rows, K, offs, vals, psi0, m, vecs, zbuf, slots, d, q, s);
-        else
-            launch_resident<TV, 9>(p, rows, K, offs, vals, psi0, m, vecs, zbuf, slots, d, q, s);
-        return check_launch(fn);
-    };
-    Resident p = resident_rows(rows, K, cu_count());
-    std::unique_lock<std::mutex> one(resident_lock(), std::defer_lock);
-    if (p.rows_per_lane && !one.try_lock()) p.rows_per_lane = 0;
-    int st = p.rows_per_lane ? resident(p) : launches_per_step();
+        st = sum_partials(pq, vtiles, q + m, stream);
+    }
     if (st) return st;
     // d and q to the host: into the caller's pinned buffer when given (the
     // copy is queued like a kernel), else through a pageable vector (the HIP
@@ -799,23 +508,10 @@ int expm_krylov(int32_t rows, int32_t cols, int32_t K, const int32_t* offs, cons
         pageable.resize(2 * (size_t)m + 1);
         hdq = pageable.data();
     }
-    auto read_back = [&]() -> int {
-        const int rc = check_hip(hipMemcpyAsync(hdq, d, sizeof(double) * (2 * (size_t)m + 1),
-                                                hipMemcpyDeviceToHost, s), fn);
-        return rc ? rc : check_hip(hipStreamSynchronize(s), fn);
-    };
-    st = read_back();
+    st = check_hip(hipMemcpyAsync(hdq, d, sizeof(double) * (2 * (size_t)m + 1),
+                                  hipMemcpyDeviceToHost, s), fn);
+    if (!st) st = check_hip(hipStreamSynchronize(s), fn);
     if (st) return st;
-    if (p.rows_per_lane) {
-        one.unlock();
-        uint64_t last;
-        std::memcpy(&last, hdq + 2 * m, sizeof(last));
-        if (last == kUnset) {   // a workgroup waited in vain
-            st = launches_per_step();
-            if (!st) st = read_back();
-            if (st) return st;
-        }
-    }
     const double* hd = hdq;
     const double* hq = hdq + m;
 

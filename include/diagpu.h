@@ -134,16 +134,17 @@ typedef struct diagpu_krylov_info {
 
 /* Device workspace (bytes, host out) for n x n H and m Lanczos steps:
  * m basis vectors of n complex64 plus O(n / 512) reduction scratch, and up to
- * n = 500000 two to four more vectors and exchange slots for the forms with
- * fewer launches. */
+ * n = 500000 two more vectors and partial sums for the form with one launch
+ * per step. */
 DIAGPU_API int diagpu_expm_krylov_workspace(int32_t n, int32_t m, size_t* bytes);
 
 /* psi_t = exp(-i t H) psi_0 for Hermitian H (n x n Recon, rows == cols; only
  * H's action is used, Hermitian symmetry is the caller's promise), complex64
  * psi_0 and psi_t of n elements, 1 <= m <= 64 Lanczos steps.  Two kernels per
- * step (SpMV with a fused dot product, three-term update with a fused norm; few
- * rows and diagonals: one kernel per step, or one for all steps),
- * deterministic fp64 reductions, scalars kept on the device; one stream
+ * step (SpMV with a fused dot product, three-term update with a fused norm; up
+ * to 7 diagonals and n = 500000: one kernel per step), deterministic fp64
+ * reductions (the same call gives the same bits, whatever runs beside it),
+ * scalars kept on the device; one stream
  * synchronisation after the m steps to read alpha and beta, then exp(-i t T_m)
  * e_1 on the host in fp64 and one combine kernel (async on `stream`).
  * host_scratch (optional) is a pinned host buffer (hipHostMalloc) of at least
