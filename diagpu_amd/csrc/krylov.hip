@@ -397,7 +397,7 @@ __global__ __launch_bounds__(kVB) void k_combine(const cf32* __restrict__ first,
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 struct Layout {
-    size_t vecs, pd, pq, d, q, zbuf, parts, total;   // pd: SpMV dot partials, pq: norm partials
+    size_t vecs, pd, pq, d, q, base, zbuf, parts, total;   // pd: SpMV dot partials, pq: norm partials
 };
 
 Layout layout(int64_t n, int m)
@@ -420,6 +420,7 @@ Layout layout(int64_t n, int m)
     L.d = off;   // d[m] and q[m+1] back to back: one copy to the host
     L.q = off + (size_t)m * sizeof(double);
     off += align256((size_t)(2 * m + 1) * sizeof(double));
+    L.base = off;   // what the three launches per step need
     L.zbuf = off;   // two z of the fused steps
     const bool fused = n <= kFusedRows;
     if (fused) off += align256(2 * (size_t)n * sizeof(cf32));
@@ -427,6 +428,17 @@ Layout layout(int64_t n, int m)
     if (fused) off += align256(4 * kFusedWgs * sizeof(double));
     L.total = off;
     return L;
+}
+
+int workspace_size(const char* fn, int32_t n, int32_t m, bool fused, size_t* bytes)
+{
+    if (!bytes) return fail(DIAGPU_ERR_ARG, "%s: bytes is NULL", fn);
+    if (n < 1 || m < 1 || m > kMaxSteps)
+        return fail(DIAGPU_ERR_ARG, "%s: n=%d m=%d (need n >= 1, 1 <= m <= %d)", fn, n, m,
+                    kMaxSteps);
+    const Layout L = layout(n, m);
+    *bytes = fused ? L.total : L.base;
+    return DIAGPU_OK;
 }
 
 template <typename TV>
@@ -446,9 +458,8 @@ int expm_krylov(int32_t rows, int32_t cols, int32_t K, const int32_t* offs, cons
     if (!std::isfinite(t)) return fail(DIAGPU_ERR_ARG, "%s: t is not finite", fn);
     const int64_t n = rows;
     const Layout L = layout(n, m);
-    if (ws_bytes < L.total)
-        return fail(DIAGPU_ERR_CAPACITY, "%s: workspace %zu bytes, needs %zu", fn, ws_bytes,
-                    L.total);
+    if (ws_bytes < L.base)
+        return fail(DIAGPU_ERR_CAPACITY, "%s: workspace %zu bytes, needs %zu", fn, ws_bytes, L.base);
     char* ws = static_cast<char*>(workspace);
     cf32* vecs = reinterpret_cast<cf32*>(ws + L.vecs);
     double* pd = reinterpret_cast<double*>(ws + L.pd);
@@ -465,7 +476,7 @@ int expm_krylov(int32_t rows, int32_t cols, int32_t K, const int32_t* offs, cons
     const int stiles = spmv_tiles<TV, cf32>(rows);
 
     int st;
-    if (K >= 1 && K <= kFusedMax && rows <= kFusedRows) {
+    if (K >= 1 && K <= kFusedMax && rows <= kFusedRows && ws_bytes >= L.total) {
         cf32* zbuf = reinterpret_cast<cf32*>(ws + L.zbuf);
         double* parts = reinterpret_cast<double*>(ws + L.parts);
         auto go = [&](auto km) {
@@ -569,13 +580,12 @@ extern "C" {
 
 DIAGPU_API int diagpu_expm_krylov_workspace(int32_t n, int32_t m, size_t* bytes)
 {
-    const char* fn = "diagpu_expm_krylov_workspace";
-    if (!bytes) return diagpu::fail(DIAGPU_ERR_ARG, "%s: bytes is NULL", fn);
-    if (n < 1 || m < 1 || m > diagpu::kMaxSteps)
-        return diagpu::fail(DIAGPU_ERR_ARG, "%s: n=%d m=%d (need n >= 1, 1 <= m <= %d)", fn, n, m,
-                            diagpu::kMaxSteps);
-    *bytes = diagpu::layout(n, m).total;
-    return DIAGPU_OK;
+    return diagpu::workspace_size("diagpu_expm_krylov_workspace", n, m, false, bytes);
+}
+
+DIAGPU_API int diagpu_expm_krylov_workspace_fused(int32_t n, int32_t m, size_t* bytes)
+{
+    return diagpu::workspace_size("diagpu_expm_krylov_workspace_fused", n, m, true, bytes);
 }
 
 DIAGPU_API int diagpu_expm_krylov_c64(const diagpu_recon_view_c64* H,

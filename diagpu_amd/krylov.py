@@ -34,7 +34,7 @@ class KrylovWorkspace:
 
     def __init__(self, n: int, m: int, device="cuda"):
         b = C.c_size_t(0)
-        _lib.call("diagpu_expm_krylov_workspace", n, m, C.byref(b))
+        _lib.call("diagpu_expm_krylov_workspace_fused", n, m, C.byref(b))
         self.n, self.m = n, m
         self.buf = torch.empty(b.value, dtype=torch.uint8, device=device)
         self.host = torch.empty(2 * m + 1, dtype=torch.float64, pin_memory=True)

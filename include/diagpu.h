@@ -133,17 +133,19 @@ typedef struct diagpu_krylov_info {
 } diagpu_krylov_info;
 
 /* Device workspace (bytes, host out) for n x n H and m Lanczos steps:
- * m basis vectors of n complex64 plus O(n / 512) reduction scratch, and up to
- * n = 500000 two more vectors and partial sums for the form with one launch
- * per step. */
+ * m basis vectors of n complex64 plus O(n / 512) reduction scratch.  _fused:
+ * up to n = 500000 two more vectors and partial sums, with which a call runs
+ * one kernel per step instead of three (the same size above). */
 DIAGPU_API int diagpu_expm_krylov_workspace(int32_t n, int32_t m, size_t* bytes);
+DIAGPU_API int diagpu_expm_krylov_workspace_fused(int32_t n, int32_t m, size_t* bytes);
 
 /* psi_t = exp(-i t H) psi_0 for Hermitian H (n x n Recon, rows == cols; only
  * H's action is used, Hermitian symmetry is the caller's promise), complex64
  * psi_0 and psi_t of n elements, 1 <= m <= 64 Lanczos steps.  Two kernels per
  * step (SpMV with a fused dot product, three-term update with a fused norm; up
- * to 7 diagonals and n = 500000: one kernel per step), deterministic fp64
- * reductions (the same call gives the same bits, whatever runs beside it),
+ * to 7 diagonals and n = 500000, with a workspace of the _fused size: one
+ * kernel per step), deterministic fp64 reductions (the same call gives the
+ * same bits, whatever runs beside it),
  * scalars kept on the device; one stream
  * synchronisation after the m steps to read alpha and beta, then exp(-i t T_m)
  * e_1 on the host in fp64 and one combine kernel (async on `stream`).

@@ -34,7 +34,7 @@ public:
     KrylovPropagator(int32_t n, int32_t max_steps) : n_(n), m_(max_steps)
     {
         size_t bytes = 0;
-        check(diagpu_expm_krylov_workspace(n, max_steps, &bytes));
+        check(diagpu_expm_krylov_workspace_fused(n, max_steps, &bytes));
         ws_.resize(bytes);
         double* h = nullptr;   // pinned: T_m's entries come back without a staged copy
         check_hip(hipHostMalloc(reinterpret_cast<void**>(&h), (2 * static_cast<size_t>(max_steps) + 1) * sizeof(double)),

@@ -273,6 +273,24 @@ def test_symbolic_noalloc_rejects_beyond_scratch():
                                               None) == _lib.ERR_ARG
 
 
+@pytest.mark.parametrize("n", [1, 511, 20000, 500000, 500001, 1 << 22])
+def test_krylov_workspace_sizes(n):
+    """The size that a caller may have kept: m basis vectors, a partial sum per
+    512 rows for the dot and for the norm, T_m's entries; the one-kernel steps
+    ask for more up to n = 500000, by their own query."""
+    up = lambda b: -(-b // 256) * 256
+    b, f = C.c_size_t(0), C.c_size_t(0)
+    for m in (1, 30, 64):
+        assert _status("diagpu_expm_krylov_workspace", n, m, C.byref(b)) == _lib.OK
+        tiles = -(-n // 512)
+        assert b.value == up(8 * m * n) + 2 * up(8 * tiles) + up(8 * (2 * m + 1))
+        assert _status("diagpu_expm_krylov_workspace_fused", n, m, C.byref(f)) == _lib.OK
+        assert f.value - b.value == (up(16 * n) + 32768 if n <= 500000 else 0)
+    assert _status("diagpu_expm_krylov_workspace_fused", 0, 1, C.byref(f)) == _lib.ERR_ARG
+    assert _status("diagpu_expm_krylov_workspace_fused", 1, 65, C.byref(f)) == _lib.ERR_ARG
+    assert _status("diagpu_expm_krylov_workspace_fused", 1, 1, None) == _lib.ERR_ARG
+
+
 def test_package_modules_import():
     """Every module of the package imports on a host without a GPU (the GPU
     tests would otherwise be the first to meet a broken module)."""

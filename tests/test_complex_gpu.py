@@ -304,6 +304,35 @@ def test_propagator_launch_forms(dev, n, pos, complex_values):
         assert abs(r.alpha[0] - a1) <= 1e-6 and abs(r.beta[0] - b1) <= 1e-6
 
 
+@pytest.mark.parametrize("n", [257, 20000])
+def test_propagator_in_the_smaller_workspace(dev, n):
+    """A workspace without the one-kernel steps' part is accepted, to the byte,
+    and gives the same psi to rounding (12 steps of a few units of 2^-24)."""
+    import ctypes as C
+
+    from diagpu_amd import _lib
+    g = torch.Generator(device=dev).manual_seed(n)
+    o = torch.tensor([16, 0, -16], dtype=torch.int32, device=dev)
+    up = torch.rand(n, generator=g, device=dev) - 0.5
+    dn = torch.zeros(n, device=dev)
+    dn[:n - 16] = up[16:]
+    v = torch.cat([up, torch.rand(n, generator=g, device=dev), dn])
+    psi0 = torch.complex(torch.randn(n, generator=g, device=dev),
+                         torch.randn(n, generator=g, device=dev))
+    ws = KrylovWorkspace(n, 12, dev)
+    full = expm_krylov(o, v, n, psi0, 0.5, 12, workspace=ws)
+    b = C.c_size_t(0)
+    _lib.call("diagpu_expm_krylov_workspace", n, 12, C.byref(b))
+    ws.buf = torch.empty(b.value, dtype=torch.uint8, device=dev)
+    small = expm_krylov(o, v, n, psi0, 0.5, 12, workspace=ws)
+    assert small.steps == full.steps
+    err = torch.linalg.vector_norm(small.psi - full.psi) / torch.linalg.vector_norm(full.psi)
+    assert err.item() <= 2e-6
+    ws.buf = ws.buf[:-1]
+    with pytest.raises(_lib.DiagpuError):
+        expm_krylov(o, v, n, psi0, 0.5, 12, workspace=ws)
+
+
 def test_propagator_from_two_threads(dev):
     """Calls that overlap on two streams of one process each give the bits of a
     call alone: what runs beside a call does not choose its kernels."""
