@@ -92,6 +92,7 @@ class SpgemmPlan:
         self._rstat = C.c_int32(0)
         self.shape = _lib.SpgemmShape()
         self._full, self._auto = {}, {}
+        self._written = None
         self._sym_fn = _lib.load().diagpu_spgemm_symbolic_shape
         self._sym_args, self._sym_caps, self._sym_ops = None, None, ()
         self.symbolic()
@@ -146,10 +147,9 @@ class SpgemmPlan:
                                C.byref(self.info))
             self._sym_caps = (self.c_cap, self.p_cap)
         st = self._sym_fn(*self._sym_args, _stream_handle(self.stream))
-        inf = self.info
-        self._counts = (inf.c_ndiag, inf.c_nnz, inf.n_pairs, inf.a_extent, inf.b_extent)
         if st:
             _lib.check(st)
+        self._written = self._state()
         if self._fused:
             rs = self._rstat.value
             if rs == _lib.OK:
@@ -158,6 +158,13 @@ class SpgemmPlan:
                 self._astat = False           # B indices beyond 2^30: not this kernel
             else:
                 _lib.check(rs)
+
+    def _state(self):
+        """What tells whether the caller has written plan arrays or counts since
+        symbolic(): torch's count of writes to the buffer that the arrays are
+        views of (inference tensors keep none), and the counts."""
+        buf, inf = self._buf, self.info
+        return (0 if buf.is_inference() else buf._version, inf.c_ndiag, inf.n_pairs)
 
     # structure views (device tensors) --------------------------------------
     def c_offsets(self) -> torch.Tensor:
@@ -342,7 +349,11 @@ class SpgemmPlan:
         """Whether "auto" runs the contiguous-band kernel
         (diagpu_spgemm_full_choice: both operands hold every offset of a range
         in ascending order, they fit in LDS, and each C diagonal takes enough
-        entries): it then stands in for the kernel that kernel_for names."""
+        entries): it then stands in for the kernel that kernel_for names.  Not
+        for a plan whose arrays or counts the caller has changed: that kernel
+        reads no entries."""
+        if self._state() != self._written:
+            return False
         v = self._full.get(dtype)
         if v is None:
             inf = self.info
@@ -361,6 +372,16 @@ class SpgemmPlan:
         if self.uses_astat(dtype):
             return "astat"
         return "gather"
+
+    def _auto_kernel(self, dtype) -> str:
+        """The kernel "auto" runs, kept while nothing it depends on changes."""
+        state = lambda: (self._state(), self._astat is True, self._band is None)
+        kept = self._auto.get(dtype)
+        if kept is not None and kept[0] == state():
+            return kept[1]
+        kernel = "full" if self.uses_full(dtype) else self.kernel_for(dtype)
+        self._auto[dtype] = (state(), kernel)
+        return kernel
 
     def numeric(self, A_vals: torch.Tensor, B_vals: torch.Tensor, C_vals: torch.Tensor,
                 kernel: str = "auto") -> None:
@@ -381,21 +402,22 @@ class SpgemmPlan:
         _check_dev(A_vals, dt, "A_vals")
         _check_dev(B_vals, dt, "B_vals")
         _check_dev(C_vals, dt, "C_vals")
-        c_ndiag, c_nnz, n_pairs, a_extent, b_extent = self._counts
+        # read at each call: a caller may have changed the plan
+        inf = self.info
+        c_ndiag, c_nnz, n_pairs = inf.c_ndiag, inf.c_nnz, inf.n_pairs
+        a_extent, b_extent = inf.a_extent, inf.b_extent
         if A_vals.numel() < a_extent or B_vals.numel() < b_extent:
             raise ValueError(f"A_vals / B_vals hold {A_vals.numel()} / {B_vals.numel()} values; "
                              f"the plan's operands need {a_extent} / {b_extent}")
         if C_vals.numel() < c_nnz:
             raise ValueError(f"C_vals has {C_vals.numel()} elements, needs {c_nnz}")
         if kernel == "auto":
-            kernel = self._auto.get(dt)
-            if kernel is None:
-                kernel = "full" if self.uses_full(dt) else self.kernel_for(dt)
-                self._auto[dt] = kernel
+            kernel = self._auto_kernel(dt)
+        elif kernel == "full" and (not self.shape.contiguous or self._state() != self._written):
+            raise ValueError("the full kernel takes contiguous bands in ascending order, with "
+                             "the plan as built")
         lib = _lib.load()
         if kernel == "full":
-            if not self.shape.contiguous:
-                raise ValueError("the full kernel takes contiguous bands in ascending order")
             A, B = self.A, self.B
             st = getattr(lib, names[2])(
                 self.n, self.shape.a_off_min, A.offsets.numel(), A.starts.data_ptr(),
@@ -419,6 +441,8 @@ class SpgemmPlan:
             return
         if kernel == "astat":
             at = self._at
+            if self._astat is True and self._state() != self._written:
+                self._astat = None          # the symbolic call's records: of another plan
             rec = at["records"] if self._astat is True else self.astat_records().data_ptr()
             A = self.A
             st = getattr(lib, names[1])(
@@ -472,6 +496,8 @@ class SpgemmPlan:
         if (self.A.offsets.numel() > cap or not 4096 <= self.n < 1 << 30
                 or inf.c_ndiag >= 1 << 29 or inf.n_pairs >= 1 << 28):
             raise ValueError("numeric_scaled: the A-stationary kernel does not take this plan")
+        if self._astat is True and self._state() != self._written:
+            self._astat = None
         if self._astat is not True:
             try:
                 self.astat_records()

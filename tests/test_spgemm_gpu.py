@@ -832,6 +832,29 @@ def test_empty_c_diagonals_written_as_zero(dev, n):
         assert np.array_equal(got.view(np.int32), want.view(np.int32)), kernel
 
 
+@pytest.mark.parametrize("n", [3000, 5000, 1 << 17])
+def test_changed_plan_is_followed_after_a_first_product(dev, n):
+    """A plan changed after "auto" has run once (on the contiguous-band kernel,
+    which reads no entries): the next products follow the entries, and the
+    contiguous-band kernel refuses it; rebuilt, it runs again."""
+    A = workloads.hm_random(n, list(range(-10, 11)), 53, dev)
+    B = workloads.hm_random(n, list(range(-8, 9)), 54, dev)
+    plan = SpgemmPlan(A, B)
+    before = plan.multiply(A.values, B.values)
+    assert plan.uses_full()
+    c_st, c_len = plan.c_starts().tolist(), plan.c_lengths().tolist()
+    _drop_diagonals(plan, [4])
+    want = before.clone()
+    want[c_st[4]: c_st[4] + c_len[4]] = 0.0
+    assert not plan.uses_full()
+    assert torch.equal(plan.multiply(A.values, B.values).view(torch.int32), want.view(torch.int32))
+    with pytest.raises(ValueError):
+        plan.multiply(A.values, B.values, kernel="full")
+    plan.symbolic()
+    assert plan.uses_full()
+    assert torch.equal(plan.multiply(A.values, B.values), before)
+
+
 def test_plan_with_no_entries(dev):
     """A plan whose every C diagonal is empty: all of C is written as 0."""
     n = 3000
