@@ -332,6 +332,18 @@ class _HostPlans:
                   self.host[s.c_off: s.c_off + 4 * s.c_ndiag].view(torch.int32).tolist())
 
 
+def _queue_offsets(H: HM, stream) -> torch.Tensor:
+    """H's offsets as the device holds them, in a pinned tensor that is filled
+    once `stream` has reached this point: the host plans come from the list
+    that H carries, which a caller may have left behind when it changed the
+    device's.  (Counts would tell most of such lists, but not all: {-5, 1, 5}
+    and {-5, -1, 5} agree in every count of their products.)"""
+    seen = torch.empty(H.offsets.numel(), dtype=torch.int32, pin_memory=True)
+    with torch.cuda.stream(stream):
+        seen.copy_(H.offsets, non_blocking=True)
+    return seen
+
+
 def power(H: HM, k: int, stats: ChainStats | None = None) -> HM:
     """H^k (k >= 1) by the chain P_j = H * P_{j-1} (P_{j-1} * H for complex
     values when H is too wide for the complex A-stationary kernel; the
@@ -349,8 +361,9 @@ def power(H: HM, k: int, stats: ChainStats | None = None) -> HM:
 def _power_steps(H: HM, k: int) -> HM:
     """power() without a wait between the products.  The first product is
     planned on the device, which checks H; the others' plans follow from its
-    offsets on the host (_HostPlans).  Where a product is not the
-    A-stationary kernel's, each plan is built on the side stream while the
+    offsets on the host (_HostPlans), read back with the first plan's counts
+    and compared with the list that H carries.  Where a product is not the
+    A-stationary kernel's, or that list was another, each plan is built on the side stream while the
     previous product runs (as _taylor_steps): a plan needs only the operands'
     structure, and P_{j-1}'s is the previous plan's C arrays, complete once
     its symbolic phase has returned.  Products stay on the caller's stream, in
@@ -360,16 +373,23 @@ def _power_steps(H: HM, k: int) -> HM:
     if k >= 3 and _narrow_first(H):
         ho = _host_offsets(H)
         plans = _HostPlans(H, _sumset(H.n, ho, ho), k - 2)
+        if not plans.ok:
+            plans = None
     side = _side_stream(H.values.device)
     side.wait_stream(main)                      # H's structure
     narrow = _narrow_first(H)
     _host_offsets(H)
+    seen = _queue_offsets(H, side) if plans is not None else None
     P = H
     for _ in range(k - 1):
         with torch.cuda.stream(side):
             plan = SpgemmPlan(H, P, stream=side) if narrow else SpgemmPlan(P, H, stream=side)
             plan.prepare(H.values.dtype)
         plan.hand_over(main)
+        if seen is not None:                    # complete since the plan's sync
+            now, seen = seen.tolist(), None
+            if now != H.host_offsets:
+                H.host_offsets, plans = now, None
         inf = plan.info
         C = HM(H.n, plan.c_offsets(), plan.c_lengths(), plan.c_starts(),
                _c_values(inf.c_nnz, H.values))
@@ -378,7 +398,7 @@ def _power_steps(H: HM, k: int) -> HM:
                 plan.numeric(H.values, P.values, C.values)
             else:
                 plan.numeric(P.values, H.values, C.values)
-        if plans is not None and plans.ok:
+        if plans is not None:
             v = C.values
             for t in range(1, k - 1):
                 v = plans.product(t, v)
@@ -433,7 +453,7 @@ def taylor_expm(H: HM, t, order: int, stats: ChainStats | None = None) -> HM:
     (fp32 bit for bit, complex to rounding)."""
     if order < 0:
         raise ValueError("order must be >= 0")
-    dev = H.values.device
+    dev, given = H.values.device, H
     if isinstance(t, complex):
         H = as_complex(H)
     if order == 0:
@@ -445,7 +465,12 @@ def taylor_expm(H: HM, t, order: int, stats: ChainStats | None = None) -> HM:
     ready.record(torch.cuda.current_stream(dev))
     S = _timed(ax, axpby, t / order, H, 1.0, _unit(H.n, dev, H.values.dtype))
     if stats is None:
-        return _taylor_steps(H, t, order, S, ready)
+        U = _taylor_steps(H, t, order, S, ready)
+        if U is None:                            # H's list was not the device's: S again
+            given.host_offsets = H.host_offsets
+            S = axpby(t / order, H, 1.0, _unit(H.n, dev, H.values.dtype))
+            U = _taylor_steps(H, t, order, S, ready, host_plans=False)
+        return U
     for j in range(order - 1, 0, -1):
         S = _horner_step_synced(H, t / j, S, stats)
     return S
@@ -521,11 +546,14 @@ def _side_stream(device) -> torch.cuda.Stream:
     return st
 
 
-def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event) -> HM:
+def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event,
+                  host_plans: bool = True) -> HM | None:
     """The Horner steps of taylor_expm without a wait between the products.
     The first is planned on the device, which checks H; the others' plans
-    follow from its offsets on the host (_HostPlans).  Where a step is not a
-    fused product, each product's plan is built on a side stream while the
+    follow from its offsets on the host (_HostPlans, unless `host_plans` is
+    False), read back with the first plan's counts.  Where the list that H
+    carried was another, H gets the device's and None is returned: S was
+    formed with the old one.  Where a step is not a fused product, each product's plan is built on a side stream while the
     previous product runs: a plan needs only its operands' structure (the
     previous plan's C arrays, complete once its symbolic phase has returned),
     so its one stream sync waits for its own symbolic phase, not for the
@@ -539,7 +567,7 @@ def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event) -> HM:
     # the steps after the first, planned on the host where they are all fused
     # products with I on their main diagonals
     plans = None
-    if order >= 3 and _narrow_first(H):
+    if host_plans and order >= 3 and _narrow_first(H):
         plans = _HostPlans(H, _sumset(H.n, _host_offsets(H), _host_offsets(S)), order - 2)
         if not (plans.ok and all(s.has_main for s in plans.steps)):
             plans = None
@@ -548,12 +576,18 @@ def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event) -> HM:
     else:
         side.wait_stream(main)                  # S's structure, formed on main
     narrow = _narrow_first(H)
+    seen = _queue_offsets(H, side) if plans is not None else None
     for j in range(order - 1, 0, -1):
         # the plan needs the operands' structure only: H's is (t/j) H's
         with torch.cuda.stream(side):
             plan = SpgemmPlan(H, S, stream=side) if narrow else SpgemmPlan(S, H, stream=side)
             fused = narrow and _fused(plan, H)   # the kernel's set-up, on the side stream
         plan.hand_over(main)
+        if seen is not None:                    # complete since the plan's sync
+            now, seen = seen.tolist(), None
+            if now != H.host_offsets:
+                H.host_offsets = now
+                return None
         inf = plan.info
         C = HM(H.n, plan.c_offsets(), plan.c_lengths(), plan.c_starts(),
                _c_values(inf.c_nnz, H.values))

@@ -415,6 +415,29 @@ def test_chain_still_refuses_wrong_lengths(dev):
         chain.taylor_expm(H, 0.1, 4)
 
 
+# An HM whose device offsets are not the list it carries: the list of another
+# set with the same lengths and the same counts of every product; one of more
+# diagonals; one without the main diagonal, or with one that the device has not.
+@pytest.mark.parametrize("offs,stale", [
+    ([-5, -1, 5], [-5, 1, 5]), ([-70, -1, 0, 1, 70], [-70, -2, 0, 2, 70]),
+    ([-70, -1, 0, 1, 70], [-71, 0, 70]), ([-70, -1, 0, 1, 70], [-70, -1, 1, 2, 70]),
+    ([-70, -1, 2, 70], [-70, 0, 2, 70]), ([-70, 0, 70], sorted({-41, 0, *range(-40, 41, 3)}))])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_chain_of_a_stale_host_list(dev, offs, stale, cplx):
+    t = 0.3 - 0.2j if cplx else 0.3
+    make = lambda host: workloads.HM(*(getattr(G, f) for f in
+                                       ("n", "offsets", "lengths", "starts", "values")), host)
+    for n in (5000, 70001):
+        G = workloads.hm_random(n, offs, seed=n, device=dev)
+        for got, want in ((chain.power(make(list(stale)), 4), chain.power(make(None), 4)),
+                          (chain.taylor_expm(make(list(stale)), t, 4),
+                           chain.taylor_expm(make(None), t, 4))):
+            assert got.offsets.tolist() == want.offsets.tolist() == got.host_offsets
+            assert torch.equal(got.starts, want.starts)
+            scale = want.values.abs().max().item()     # device plans: unfused steps may differ
+            assert (got.values - want.values).abs().max().item() <= 1e-5 * scale
+
+
 def test_power_of_unordered_offsets(dev):
     """Offsets in descending order: planned on the device, as before."""
     A = workloads.hm_random(5000, [-70, -1, 0, 1, 70], seed=4, device=dev)
