@@ -332,16 +332,28 @@ class _HostPlans:
                   self.host[s.c_off: s.c_off + 4 * s.c_ndiag].view(torch.int32).tolist())
 
 
-def _queue_offsets(H: HM, stream) -> torch.Tensor:
-    """H's offsets as the device holds them, in a pinned tensor that is filled
-    once `stream` has reached this point: the host plans come from the list
-    that H carries, which a caller may have left behind when it changed the
-    device's.  (Counts would tell most of such lists, but not all: {-5, 1, 5}
-    and {-5, -1, 5} agree in every count of their products.)"""
-    seen = torch.empty(H.offsets.numel(), dtype=torch.int32, pin_memory=True)
-    with torch.cuda.stream(stream):
-        seen.copy_(H.offsets, non_blocking=True)
-    return seen
+class _DeviceOffsets:
+    """H's offsets as the device holds them, on their way to the host: the host
+    plans come from the list that H carries, which a caller may have left
+    behind when it changed the device's.  (Counts would tell most of such
+    lists, but not all: {-5, 1, 5} and {-5, -1, 5} agree in every count of
+    their products.)  The copy runs on the caller's stream, beside the first
+    plan on the side stream."""
+
+    def __init__(self, H: HM):
+        self.seen = torch.empty(H.offsets.numel(), dtype=torch.int32, pin_memory=True)
+        self.seen.copy_(H.offsets, non_blocking=True)
+        self.copied = torch.cuda.Event()
+        self.copied.record()
+
+    def differ(self, H: HM) -> bool:
+        """Whether they are not H's list, which they replace then."""
+        self.copied.synchronize()
+        now = self.seen.tolist()
+        if now == H.host_offsets:
+            return False
+        H.host_offsets = now
+        return True
 
 
 def power(H: HM, k: int, stats: ChainStats | None = None) -> HM:
@@ -361,13 +373,13 @@ def power(H: HM, k: int, stats: ChainStats | None = None) -> HM:
 def _power_steps(H: HM, k: int) -> HM:
     """power() without a wait between the products.  The first product is
     planned on the device, which checks H; the others' plans follow from its
-    offsets on the host (_HostPlans), read back with the first plan's counts
-    and compared with the list that H carries.  Where a product is not the
-    A-stationary kernel's, or that list was another, each plan is built on the side stream while the
-    previous product runs (as _taylor_steps): a plan needs only the operands'
-    structure, and P_{j-1}'s is the previous plan's C arrays, complete once
-    its symbolic phase has returned.  Products stay on the caller's stream, in
-    order."""
+    offsets on the host (_HostPlans), if the list that H carries is what the
+    device holds (_DeviceOffsets).  Where a product is not the A-stationary
+    kernel's, or the list was another, each plan is built on the side stream
+    while the previous product runs (as _taylor_steps): a plan needs only the
+    operands' structure, and P_{j-1}'s is the previous plan's C arrays,
+    complete once its symbolic phase has returned.  Products stay on the
+    caller's stream, in order."""
     main = torch.cuda.current_stream(H.values.device)
     plans = None
     if k >= 3 and _narrow_first(H):
@@ -379,17 +391,13 @@ def _power_steps(H: HM, k: int) -> HM:
     side.wait_stream(main)                      # H's structure
     narrow = _narrow_first(H)
     _host_offsets(H)
-    seen = _queue_offsets(H, side) if plans is not None else None
+    check = _DeviceOffsets(H) if plans is not None else None
     P = H
     for _ in range(k - 1):
         with torch.cuda.stream(side):
             plan = SpgemmPlan(H, P, stream=side) if narrow else SpgemmPlan(P, H, stream=side)
             plan.prepare(H.values.dtype)
         plan.hand_over(main)
-        if seen is not None:                    # complete since the plan's sync
-            now, seen = seen.tolist(), None
-            if now != H.host_offsets:
-                H.host_offsets, plans = now, None
         inf = plan.info
         C = HM(H.n, plan.c_offsets(), plan.c_lengths(), plan.c_starts(),
                _c_values(inf.c_nnz, H.values))
@@ -398,6 +406,8 @@ def _power_steps(H: HM, k: int) -> HM:
                 plan.numeric(H.values, P.values, C.values)
             else:
                 plan.numeric(P.values, H.values, C.values)
+        if plans is not None and check.differ(H):   # while the product runs
+            plans = None
         if plans is not None:
             v = C.values
             for t in range(1, k - 1):
@@ -551,9 +561,9 @@ def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event,
     """The Horner steps of taylor_expm without a wait between the products.
     The first is planned on the device, which checks H; the others' plans
     follow from its offsets on the host (_HostPlans, unless `host_plans` is
-    False), read back with the first plan's counts.  Where the list that H
-    carried was another, H gets the device's and None is returned: S was
-    formed with the old one.  Where a step is not a fused product, each product's plan is built on a side stream while the
+    False).  Where the list that H carried is not what the device holds
+    (_DeviceOffsets), H gets the device's and None is returned: S was formed
+    with the old one.  Where a step is not a fused product, each product's plan is built on a side stream while the
     previous product runs: a plan needs only its operands' structure (the
     previous plan's C arrays, complete once its symbolic phase has returned),
     so its one stream sync waits for its own symbolic phase, not for the
@@ -576,18 +586,13 @@ def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event,
     else:
         side.wait_stream(main)                  # S's structure, formed on main
     narrow = _narrow_first(H)
-    seen = _queue_offsets(H, side) if plans is not None else None
+    check = _DeviceOffsets(H) if plans is not None else None
     for j in range(order - 1, 0, -1):
         # the plan needs the operands' structure only: H's is (t/j) H's
         with torch.cuda.stream(side):
             plan = SpgemmPlan(H, S, stream=side) if narrow else SpgemmPlan(S, H, stream=side)
             fused = narrow and _fused(plan, H)   # the kernel's set-up, on the side stream
         plan.hand_over(main)
-        if seen is not None:                    # complete since the plan's sync
-            now, seen = seen.tolist(), None
-            if now != H.host_offsets:
-                H.host_offsets = now
-                return None
         inf = plan.info
         C = HM(H.n, plan.c_offsets(), plan.c_lengths(), plan.c_starts(),
                _c_values(inf.c_nnz, H.values))
@@ -604,6 +609,8 @@ def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event,
                 else:
                     plan.numeric(S.values, Hj.values, C.values)
             sigma = 0.0
+        if plans is not None and j == order - 1 and check.differ(H):   # while the product runs
+            return None
         if plans is not None and sigma and j == order - 1:
             v = C.values
             for t_ in range(1, order - 1):
