@@ -208,7 +208,7 @@ def multiply(A: HM, B: HM, stats: ChainStats | None = None) -> HM:
         torch.cuda.synchronize()
     t0 = time.perf_counter()
     plan = SpgemmPlan(A, B)
-    plan.prepare(A.values.dtype)      # the numeric kernel's set-up belongs to the plan
+    plan._auto_kernel(A.values.dtype)   # the numeric kernel's set-up belongs to the plan
     inf = plan.info
     # C's structure arrays are views of the plan's buffer (kept alive by
     # them)
@@ -396,7 +396,7 @@ def _power_steps(H: HM, k: int) -> HM:
     for _ in range(k - 1):
         with torch.cuda.stream(side):
             plan = SpgemmPlan(H, P, stream=side) if narrow else SpgemmPlan(P, H, stream=side)
-            plan.prepare(H.values.dtype)
+            plan._auto_kernel(H.values.dtype)   # the numeric kernel's set-up
         plan.hand_over(main)
         inf = plan.info
         C = HM(H.n, plan.c_offsets(), plan.c_lengths(), plan.c_starts(),

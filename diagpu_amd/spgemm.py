@@ -186,10 +186,13 @@ class SpgemmPlan:
     # streams -----------------------------------------------------------------
     def prepare(self, dtype=torch.float32) -> str:
         """Runs now, on the plan's stream, the per-plan set-up of the kernel
-        `numeric` takes by default for `dtype` (band or A-stationary
-        prepare, each one stream sync; none for "full"), and returns that
-        kernel's name."""
-        return "full" if self.uses_full(dtype) else self.kernel_for(dtype)
+        that kernel_for names for `dtype` (band or A-stationary prepare, each
+        one stream sync), and returns the name of the kernel `numeric` takes
+        by default: that one, or "full" where the contiguous-band kernel,
+        which needs no set-up, stands in for it.  Neither then waits for the
+        stream in numeric (so both can be captured)."""
+        general = self.kernel_for(dtype)
+        return "full" if self.uses_full(dtype) else general
 
     def hand_over(self, stream) -> None:
         """Continue the plan on `stream` (a torch stream): its buffers are

@@ -88,3 +88,20 @@ def test_contiguous_band_kernel_only_for_the_plan_as_built(plan):
     assert _numeric(plan, "auto")[0] == "diagpu_spgemm_numeric_full_f32"
     plan.info.n_pairs = 8                    # counts changed
     assert _numeric(plan, "auto")[0] == "diagpu_spgemm_numeric_astat_f32"
+
+
+def test_prepare_leaves_no_set_up_to_the_general_kernel(plan, monkeypatch):
+    """prepare() on a contiguous band: the kernel that kernel_for names has its
+    set-up too, so forcing it later waits for nothing."""
+    def eligible(n, *args):
+        args[-2]._obj.eligible = 1
+        return 0
+    plan.n = 1 << 18
+    monkeypatch.setattr(plan.test_lib, "diagpu_spgemm_band_prepare", eligible, raising=False)
+    plan.info.n_pairs = 15                   # from 3 entries per C diagonal on
+    plan._written = plan._state()
+    plan.test_lib.info.n_pairs = 15
+    assert plan.prepare() == "full" and plan.kernel_for() == "band"
+    assert plan._band is not None and plan._band[1].eligible
+    name, _ = _numeric(plan, "band")
+    assert name == "diagpu_spgemm_numeric_band_f32"
