@@ -19,14 +19,18 @@
 // global-to-LDS loads, and one row of zeros behind each operand.  Wave w then
 // computes the k-tile w of every row of the block.  The p of each C value run
 // downwards, which is the plan's order (B ascending), one fused multiply-add
-// each: the bits of the gather kernel.  At the ends of a tile's p range some
+// each: the bits of the gather kernel, but for the sign of a zero that
+// underflow makes (below).  At the ends of a tile's p range some
 // of a group's p or q lie outside [0, nA) or [0, nB): those read the row of
 // zeros, and A elements that do not exist (rows m outside [0, n)) are staged
 // as zeros, so every group runs the same straight-line code; a product with
-// a zero leaves its sum as it is (sums start at +0 and are never -0) unless
-// the other factor is infinite or NaN, which is found afterwards and formed
-// again term by term.  (With the ends' terms behind uniform branches the
-// kernel took 34 us instead of 19 on the first shape below.)
+// a zero leaves its sum as it is unless the other factor is infinite or NaN,
+// which is found afterwards and formed again term by term, or the sum is -0.
+// Sums start at +0, and only a negative product below half the smallest
+// denormal makes one -0; a product that is +0 then makes it +0, where the
+// gather, which has no such product, keeps -0.  No other value depends on it.
+// (With the ends' terms behind uniform branches the kernel took 34 us instead
+// of 19 on the first shape below.)
 //
 // What bounds it: at 33 x 33 diagonals and n = 100000 LDS reads (21 of 16
 // bytes for 128 multiply-adds per lane at RR = 4, KT = 8) and the one round

@@ -393,7 +393,8 @@ class SpgemmPlan:
         else kernel_for), "gather" (any plan), "band" (fp32, narrow bands),
         "astat" (at most DIAGPU_ASTAT_MAX_A A diagonals,
         DIAGPU_ASTAT_MAX_A_C64 for complex values) or "full" (contiguous
-        bands in ascending order), which all return the same bits, or
+        bands in ascending order), which all return the same bits ("full" but
+        for the sign of a zero made by products that underflow), or
         "band_mfma" (fp32, narrow bands on the matrix cores: the same values
         to rounding, finite operands)."""
         dt = A_vals.dtype

@@ -468,8 +468,9 @@ DIAGPU_API int diagpu_spgemm_symbolic_shape(
     diagpu_spgemm_shape* shape,
     diagpu_spgemm_info* info, void* stream);
 
-/* The numeric phase of diagpu_spgemm_numeric_f32 / _c64 (same C, bit for bit)
- * for contiguous bands in ascending order (shape->contiguous), as
+/* The numeric phase of diagpu_spgemm_numeric_f32 / _c64 (same C, bit for bit,
+ * except that a zero made by products that underflow may be +0 where theirs is
+ * -0) for contiguous bands in ascending order (shape->contiguous), as
  * make_banded and gemm_diag have them: register tiles of C over operands
  * staged in LDS, no plan entries read.  nA + nB - 1 = c_ndiag C diagonals,
  * all sums of offsets inside (-n, n) (else DIAGPU_ERR_ARG); operands that do

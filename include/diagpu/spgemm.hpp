@@ -253,7 +253,10 @@ namespace diagpu {
 //                narrow bands only, else diagpu::Error with DIAGPU_ERR_CAPACITY);
 //   AStationary: diagpu_spgemm_numeric_astat_f32 (A held in LDS; at most
 //                DIAGPU_ASTAT_MAX_A A diagonals, else DIAGPU_ERR_CAPACITY).
-// All return the same bits.
+//   Full:        diagpu_spgemm_numeric_full_f32 (contiguous bands in ascending
+//                order, else DIAGPU_ERR_ARG).
+// All return the same bits, but for the sign of a zero made by products that
+// underflow (Full).
 enum class NumericKernel { Auto, Gather, Band, AStationary, Full };
 
 // Device-resident C = A * B for HM operands whose offsets, lengths and starts

@@ -1012,6 +1012,36 @@ def test_full_same_bits_as_gather(dev, oracle, n, a0, na, b0, nb, dtype):
         assert torch.equal(torch.nan_to_num(got, nan=0.0), torch.nan_to_num(ref, nan=0.0))
 
 
+@pytest.mark.parametrize("n,a0,na,b0,nb", [FULL_SHAPES[i] for i in (1, 6, 7, 10, 12)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.complex64])
+def test_full_where_products_underflow(dev, n, a0, na, b0, nb, dtype):
+    """Values of about 1e-30 of both signs among ordinary ones, whole diagonals
+    of them: every value is the gather's, and every bit but the sign of zeros
+    (which the zero products at a band's ends may turn from -0 to +0)."""
+    g = torch.Generator(device=dev).manual_seed(n)
+    A = workloads.hm_random(n, range(a0, a0 + na), seed=n, device=dev)
+    B = workloads.hm_random(n, range(b0, b0 + nb), seed=n + 1, device=dev)
+
+    def tiny(M):
+        v = M.values * 1e-30
+        keep = torch.rand(v.numel(), generator=g, device=dev) < 0.3
+        keep[: M.n - 1] = False                       # the first diagonal: all tiny
+        v = torch.where(keep, M.values, v)
+        return torch.complex(v, torch.roll(v, 3)).contiguous() if dtype.is_complex else v
+
+    av, bv = tiny(A), tiny(B)
+    plan = SpgemmPlan(A, B)
+    C = torch.full((plan.info.c_nnz,), float("nan"), dtype=dtype, device=dev)
+    plan.numeric(av, bv, C, kernel="full")
+    want = plan.multiply(av, bv, kernel="gather")
+    if dtype.is_complex:
+        C, want = torch.view_as_real(C), torch.view_as_real(want)
+    assert torch.equal(C, want)                       # 0 == -0
+    differ = C.view(torch.int32) != want.view(torch.int32)
+    assert not bool((differ & (want != 0)).any())
+    assert bool((want == 0).any())
+
+
 def test_full_only_for_contiguous_bands_in_order(dev):
     """Holes, another order, or sums clipped at n: the general kernels."""
     n = 70000
