@@ -30,7 +30,8 @@ import numpy as np
 import torch
 
 from . import _lib
-from .spgemm import BAND_LDS_BUDGET, BAND_ROWS, SpgemmPlan, _check_dev
+from .spgemm import (BAND_LDS_BUDGET, SpgemmPlan, _check_dev, astat_rule, band_lds_bytes,
+                     band_rule)
 from .spmv import _on_stream, _stream_handle
 from .workloads import HM, hm_layout
 
@@ -289,15 +290,12 @@ class _HostPlans:
         (uses_band, uses_full and uses_astat, from the host's counts; plans
         that may be one of the others' are left to the device path)."""
         na, np_, nc = len(ho), s.n_pairs, s.c_ndiag
-        if nc == 0 or nc >= 1 << 29 or np_ >= 1 << 28 or np_ == na * nb and nc == na + nb - 1:
+        if np_ == na * nb and nc == na + nb - 1:
             return False
-        if dt == torch.complex64:
-            return self.n >= 1 << 16 or np_ >= 3 * na
-        if np_ >= 3 * nc and self.n >= 1024 * BAND_ROWS:
-            wb = (BAND_ROWS + ho[-1] - ho[0] + 3) & ~3
-            if 4 * (na * BAND_ROWS + nb * wb) + 16 * np_ <= BAND_LDS_BUDGET:
-                return False
-        return not (np_ < 16 and 2 * np_ >= 3 * nc and 1 << 19 <= self.n < 1 << 20)
+        if (band_rule(dt, self.n, na, nb, nc, np_)
+                and band_lds_bytes(na, nb, ho[-1] - ho[0], np_) <= BAND_LDS_BUDGET):
+            return False
+        return astat_rule(dt, self.n, na, nc, np_)
 
     def product(self, t: int, B: torch.Tensor, alpha=None, sigma=0.0) -> torch.Tensor:
         """C_t's values from C_{t-1}'s: H B, or (alpha H) B + sigma I."""

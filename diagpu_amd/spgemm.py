@@ -42,6 +42,34 @@ _NUMERIC = {
 _KERNELS = frozenset(("auto", "gather", "band", "astat", "full", "band_mfma"))
 
 
+def band_lds_bytes(na: int, nb: int, a_span: int, n_pairs: int) -> int:
+    """The band kernel's LDS bytes per workgroup, as diagpu_spgemm_band_prepare
+    reports them: 4 (nA 256 + nB wb) + 16 n_pairs, wb = 256 + A's offset span
+    rounded up to a multiple of 4."""
+    wb = (BAND_ROWS + a_span + 3) & ~3
+    return 4 * (na * BAND_ROWS + nb * wb) + 16 * n_pairs
+
+
+def band_rule(dtype, n: int, na: int, nb: int, c_ndiag: int, n_pairs: int) -> bool:
+    """The automatic choice of the band kernel (SpgemmPlan.uses_band), but for
+    its LDS footprint."""
+    return (dtype == torch.float32 and c_ndiag > 0 and na <= 65535 and nb <= 32767
+            and n_pairs >= 3 * c_ndiag and n >= 1024 * BAND_ROWS)
+
+
+def astat_rule(dtype, n: int, na: int, c_ndiag: int, n_pairs: int) -> bool:
+    """The automatic choice of the A-stationary kernel after the band kernel
+    (SpgemmPlan.uses_astat), but for the range of B's indices."""
+    if c_ndiag == 0 or n < 4096 or n >= 1 << 30 or c_ndiag >= 1 << 29 or n_pairs >= 1 << 28:
+        return False
+    if dtype == torch.float32:
+        thin_mid = n_pairs < 16 and 2 * n_pairs >= 3 * c_ndiag and 1 << 19 <= n < 1 << 20
+        return na <= _lib.ASTAT_MAX_A and not thin_mid
+    if dtype == torch.complex64:
+        return na <= _lib.ASTAT_MAX_A_C64 and (n >= 1 << 16 or n_pairs >= 3 * na)
+    return False
+
+
 class SpgemmPlan:
     """C = A * B for HM operands (objects with n, offsets, lengths, starts,
     int32/int32/int64 device tensors).  Builds the C structure and pair plan
@@ -234,8 +262,7 @@ class SpgemmPlan:
         A-stationary vs band 14.5 vs 20.0 us at n = 2^17, 32.0 vs 27.9 us at
         2^18; the 9-diagonal band's square 6.3 vs 8.2 and 11.7 vs 11.1 us)."""
         na, nb = self.A.offsets.numel(), self.B.offsets.numel()
-        if (dtype != torch.float32 or self.info.c_ndiag == 0 or na > 65535 or nb > 32767
-                or self.info.n_pairs < 3 * self.info.c_ndiag or self.n < 1024 * 256):
+        if not band_rule(dtype, self.n, na, nb, self.info.c_ndiag, self.info.n_pairs):
             return False
         est = self.band_lds_estimate()
         if est is not None and est > BAND_LDS_BUDGET:
@@ -243,16 +270,13 @@ class SpgemmPlan:
         return bool(self.band_info()[1].eligible)
 
     def band_lds_estimate(self) -> int | None:
-        """The band kernel's LDS bytes per workgroup for this plan, as
-        diagpu_spgemm_band_prepare reports them (4 (nA 256 + nB wb) +
-        16 n_pairs, wb = 256 + A's offset span rounded up to a multiple of
-        4), from A's host offsets when A carries them; else None."""
+        """band_lds_bytes of this plan, from A's host offsets when A carries
+        them; else None."""
         ho = getattr(self.A, "host_offsets", None)
         if not ho:
             return None
-        span = max(ho) - min(ho)
-        wb = (BAND_ROWS + span + 3) & ~3
-        return 4 * (len(ho) * BAND_ROWS + self.B.offsets.numel() * wb) + 16 * self.info.n_pairs
+        return band_lds_bytes(len(ho), self.B.offsets.numel(), max(ho) - min(ho),
+                              self.info.n_pairs)
 
     def astat_records(self) -> torch.Tensor:
         """Records of diagpu_spgemm_astat_prepare for this plan; int32
@@ -309,20 +333,8 @@ class SpgemmPlan:
         re-reads the operand runs at its items' edges); the gather was
         faster (5.9 vs 6.3 us) on a 4096-row product with 2 entries per A
         diagonal."""
-        na = self.A.offsets.numel()
         inf = self.info
-        if (inf.c_ndiag == 0 or self.n < 4096 or self.n >= 1 << 30 or inf.c_ndiag >= 1 << 29
-                or inf.n_pairs >= 1 << 28):
-            return False
-        if dtype == torch.float32:
-            thin_mid = (inf.n_pairs < 16 and 2 * inf.n_pairs >= 3 * inf.c_ndiag
-                        and 1 << 19 <= self.n < 1 << 20)
-            ok = na <= _lib.ASTAT_MAX_A and not thin_mid
-        elif dtype == torch.complex64:
-            ok = na <= _lib.ASTAT_MAX_A_C64 and (self.n >= 1 << 16 or inf.n_pairs >= 3 * na)
-        else:
-            ok = False
-        if not ok:
+        if not astat_rule(dtype, self.n, self.A.offsets.numel(), inf.c_ndiag, inf.n_pairs):
             return False
         if self._astat is False:                  # refused before: B indices beyond 2^30
             return False
