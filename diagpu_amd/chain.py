@@ -342,7 +342,7 @@ class _DeviceOffsets:
         self.seen = torch.empty(H.offsets.numel(), dtype=torch.int32, pin_memory=True)
         self.seen.copy_(H.offsets, non_blocking=True)
         self.copied = torch.cuda.Event()
-        self.copied.record()
+        self.copied.record(torch.cuda.current_stream(H.offsets.device))
 
     def differ(self, H: HM) -> bool:
         """Whether they are not H's list, which they replace then."""

@@ -171,9 +171,12 @@ template <int BS> __device__ __forceinline__ void block_sum2(double& a, double& 
 // an update and a sum launch per step it reads z_j, u_j and u_{j-1} once for
 // both (the columns' copies come from the caches) and writes u_{j+1} and
 // z_{j+1} once: 60 instead of 68 bytes of HBM traffic a row at K = 5, and no
-// launch between them.  n = 360000 401 -> 346 us, level with the three launches at 600000 (m = 30), and slower above,
-// where the columns' 16 runs a lane through the vector L1 cost more than the
-// launches (n = 2^22: 63 us a step against 53); so it ends at kFusedRows.
+// launch between them.  Calls with m = 30 (5 diagonals, real H): n = 1024 340
+// -> 233 us, 19881 346 -> 234, 65536 347 -> 241, 262144 365 -> 290, 360000 393
+// -> 335, 499849 432 -> 399; level with the three launches at 600000, and
+// slower above, where the columns' 16 runs a lane through the vector L1 cost
+// more than the launches (n = 2^22: 63 us a step against 53); so it ends at
+// kFusedRows.
 // The grid is at most kFusedWgs workgroups, each over tiles of 512 rows of its
 // XCD's range in step with the others, so that the next launch can add all
 // parts at its start in every workgroup.

@@ -7,7 +7,6 @@
 
 namespace diagpu {
 
-// Inclusive prefix sum across the 64 lanes of a wave.
 // `x` moved between lanes by a DPP control; lanes that get nothing keep `id`.
 template <int Ctrl, int RowMask>
 __device__ __forceinline__ int32_t dpp_move(int32_t x, int32_t id)
@@ -35,6 +34,7 @@ __device__ __forceinline__ T wave_scan_dpp(T v, T id, Op op)
     return op(v, dpp_move<0x143, 0xc>(v, id));   // row_bcast:31
 }
 
+// Inclusive prefix sum across the 64 lanes of a wave.
 template <typename T>
 __device__ __forceinline__ T wave_inclusive_scan(T v)
 {
