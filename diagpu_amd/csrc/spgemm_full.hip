@@ -297,25 +297,75 @@ bool fits(FullKind kind, int nA, int nB, size_t size)
 
 // The form a launch takes (kNone: the operands do not fit in LDS).  Few rows:
 // small blocks, so that more workgroups share the work (21 x 21, n = 4096:
-// 4.8 us at 1 x 4, 6.8 at 2 x 8, 9.0 at 4 x 8; at n = 20000 7.0, 7.1, 9.5).
+// 4.8 us at 1 x 4, 6.8 at 2 x 8, 9.0 at 4 x 8), as long as every CU gets at
+// most one workgroup, 256 blocks of 64 rows, or two of few waves (fp32 33 x
+// 33 at n = 16000: 8.1 us at 1 x 4, 8.5 at 2 x 8, at 17000 10.2 and 8.5, 33 x
+// 19 at 17000 7.7 and 8.2; complex 15 x 15 at 18000 6.3 at 1 x 4 and at 2 x 4,
+// 21 x 21 8.0 and 7.4, 11 x 11 5.4 and 5.8, at 26000 5.7 and 5.8, 21 x 11 at
+// 26000 6.9 and 6.7, 9 x 9 at 40000 5.9 and 6.5, at 55000 7.0 and 6.5).
 // fp32 above: 2 x 8, and 4 x 8 where the LDS reads bound it (about 14 entries
 // per C diagonal) and two workgroups still fit a CU (33 x 33, n = 100003: 17.6
 // against 15.6; 17 x 17, n = 200003: 15.6 against 17.0).  Complex values: 2 x
-// 4 for short tiles (11 x 11, n = 300007: 19.9 us, 23.0 at 2 x 6), 2 x 6 above
+// 4 for short tiles (11 x 11, n = 300007: 19.9 us, 23.0 at 2 x 6) and, up to
+// 32768 rows, where one workgroup holds all tiles (64 C diagonals; 29 x 11 at
+// 26000 7.2 us, 8.3 at 2 x 6, 33 x 33 at 24000 16.3 and 10.6), 2 x 6 above
 // (33 x 33, n = 100003: 50.8 at 2 x 4, 37.4 at 2 x 6, 42.5 at 2 x 8).
 FullKind full_kind(int32_t n, int nA, int nB, bool cplx)
 {
     const size_t size = cplx ? sizeof(cf32) : sizeof(float);
     const int64_t pairs = (int64_t)nA * nB, nC = nA + nB - 1;
     FullKind kind;
-    if (n < 20000)
+    if (n <= 16384 || (n < 20000 && nC <= (cplx ? 32 : 52)) || (cplx && n <= 32768 && nC <= 24))
         kind = k1x4;
     else if (cplx)
-        kind = pairs < 6 * nC ? k2x4 : k2x6;
+        kind = pairs < 6 * nC || (n <= 32768 && nC <= 64) ? k2x4 : k2x6;
     else
         kind = n >= 65536 && pairs >= 14 * nC && Full<4>::lds(nA, nB, size) <= 80 * 1024 ? k4x8 : k2x8;
     if (!fits(kind, nA, nB, size)) kind = k1x4;
     return fits(kind, nA, nB, size) ? kind : kNone;
+}
+
+// Tenths of an entry per C diagonal from which this kernel is the faster one
+// (us, the general kernels against this one; -1: never).
+int full_tenths(int32_t n, int nA, int nB, bool cplx)
+{
+    const int nC = nA + nB - 1;
+    // the gather: fp32 5 x 5 (2.8) at n = 2000 5.8 / 3.3, complex 3 x 37 (2.9)
+    // 5.4 / 4.4 (the exceptions are complex 5 x 49, 37 x 5 and 49 x 5, 0.89 to
+    // 0.96 of the general kernel's rate)
+    if (n < 4096) return 25;
+    if (cplx) {
+        // 5 x 5 (2.8) at n = 5000 4.2 / 3.7; 3 x 49 (2.9) 4.7 / 5.0
+        if (n <= 10000) return 25;
+        // Each wave of the A-stationary kernel takes one C diagonal, and its
+        // blocks of 256 rows (with 32 before them) are one round of
+        // workgroups: 7 x 7 (3.8) at n = 33000 4.9 / 5.4, 55000 5.1 / 5.6, 9 x
+        // 7 (4.2) 5.6 / 6.0; past one of the two 9 x 9 (4.8) at 55000 9.0 /
+        // 6.5, 7 x 7 at 65535 6.8 / 5.7
+        if (nC <= 16 && n > 32768 && n <= 65536 - 32) return -1;
+        // 5 x 5 (2.8) at n = 100003 5.1 / 5.6; 7 x 7 (3.8) 7.0 / 6.9, 24000
+        // 4.9 / 4.4, 10^6 56 / 43; 5 x 21 (4.2) at 18000 5.6 / 5.4 (5 x 37, 4.5,
+        // loses up to 40000: 5.9 / 6.3 at 18000, 8.4 / 9.0 at 40000)
+        return 35;
+    }
+    // 7 x 7 (3.8) at 100003 4.4 / 6.4; 11 x 11 (5.8) at 300007 13.6 / 14.8; 33 x
+    // 9 (7.2) at 491830 36.0 / 37.8; 21 x 11 (7.5) at 94475 9.1 / 9.5; 15 x 15
+    // (7.8) at 300007 19.7 / 18.0, 100003 10.7 / 9.5
+    if (n >= 65536) return 76;
+    // more than 64 C diagonals are two workgroups per 64 rows, from 8192 rows
+    // on more than one per CU: 21 x 49 (14.9) at n = 9999 7.6 / 8.0, 17 x 49
+    // (12.8) at 12500 6.8 / 7.5, 33 x 33 (16.8) 9.3 / 8.0; at 15000, where the
+    // A-stationary kernel takes a second round, 21 x 49 9.0 / 8.3
+    if (nC > 64 && n > 8192 && n < 15000) return 150;
+    // 21 x 21 (10.8) at n = 20000 6.2 / 7.0; 17 x 39 (12.1) 8.7 / 7.7; 33 x 25
+    // (14.5) at 30011 11.5 / 8.5
+    if (n > 10000) return 120;
+    // latency: a launch's waves grow with the C diagonals, the general
+    // kernels' time with the entries.  At n = 4200: 5 x 5 (2.8) 3.4 / 3.3, 7 x 5
+    // (3.2) 3.3 / 3.5, 3 x 29 (2.8) 3.5 / 3.7, 7 x 7 (3.8) 3.6 / 3.5, 5 x 29
+    // (4.4) 3.9 / 3.8; 5 x 37 (4.5) 3.9 / 4.3, 3 x 49 (2.9) 3.5 / 4.7, 7 x 37
+    // (6.0) 4.3 / 4.5, 37 x 7 4.9 / 4.8, 9 x 37 (7.4) 4.8 / 4.5
+    return nC <= 9 ? 25 : nC <= 36 ? 33 : nB > nA ? 70 : 60;
 }
 
 template <typename T, int RR, int KT>
@@ -397,18 +447,8 @@ DIAGPU_API int diagpu_spgemm_full_choice(int32_t n, int32_t nA, int32_t nB, int6
         !inside_n(n, (int64_t)shape->a_off_min + shape->b_off_min, nC))
         return 0;
     if (full_kind(n, nA, nB, complex_values != 0) == kNone) return 0;
-    // Entries per C diagonal from which this kernel is the faster one (us, the
-    // general kernels against this one):
-    //   n <= 10000 (few workgroups: latency): 5 x 5 (2.8) 4.9 against 3.3, 9 x
-    //     9 (4.8) 4.3 / 3.7; complex 5 x 5 4.2 / 3.7
-    //   complex: 5 x 5 (2.8) at n = 100003 5.1 / 5.6; 7 x 7 (3.8) 7.4 / 6.8,
-    //     10^6 56 / 43
-    //   fp32 from n = 65536: 7 x 7 (3.8) at 100003 4.4 / 6.4; 11 x 11 (5.8) at
-    //     300007 13.6 / 14.8; 15 x 15 (7.8) 19.7 / 18.0, 100003 10.7 / 9.5
-    //   fp32 between: 21 x 21 (10.8) at n = 20000 6.4 / 7.1; 33 x 25 (14.5) at
-    //     30011 11.5 / 8.5
-    const int64_t tenths = n <= 10000 ? 25 : complex_values ? 35 : n >= 65536 ? 70 : 120;
-    return 10 * pairs >= tenths * nC ? 1 : 0;
+    const int tenths = full_tenths(n, nA, nB, complex_values != 0);
+    return tenths >= 0 && 10 * pairs >= tenths * nC ? 1 : 0;
 }
 
 DIAGPU_API int diagpu_spgemm_numeric_full_f32(int32_t n, int32_t a_off_min, int32_t nA,

@@ -326,6 +326,26 @@ def test_full_choice_is_host_logic():
     assert fn(100, 3, 3, 5, 9, None, 0) == 0
 
 
+@pytest.mark.parametrize("n,na,nb,cplx,full", [
+    # fp32 below 10000 rows: wide C of few entries stays with the general kernels
+    (4200, 3, 49, 0, 0), (9999, 5, 37, 0, 0), (8000, 49, 5, 0, 0), (4200, 7, 5, 0, 0),
+    (4200, 7, 37, 0, 0), (4200, 37, 7, 0, 1), (4200, 7, 7, 0, 1), (4200, 5, 29, 0, 1),
+    (4095, 3, 49, 0, 1), (4200, 9, 37, 0, 1), (4096, 21, 21, 0, 1),
+    # more than 64 C diagonals in more workgroups than CUs
+    (8192, 17, 49, 0, 1), (8193, 17, 49, 0, 0), (14999, 21, 49, 0, 0), (15000, 21, 49, 0, 1),
+    (12500, 33, 33, 0, 1), (9000, 17, 48, 0, 1), (17000, 17, 49, 0, 1),
+    (94475, 21, 11, 0, 0), (100003, 15, 15, 0, 1),
+    # complex: one C diagonal per wave of the A-stationary kernel, one round of blocks
+    (32768, 7, 7, 1, 1), (32769, 7, 7, 1, 0), (65504, 9, 8, 1, 0), (65505, 9, 8, 1, 1),
+    (50000, 9, 9, 1, 1)])
+def test_full_choice_where_the_general_kernels_are_faster(n, na, nb, cplx, full):
+    """The measured lines of the automatic choice, on both sides."""
+    a0, b0 = -(na // 2), -(nb // 2)
+    sh = _lib.SpgemmShape(a0, a0 + na - 1, b0, b0 + nb - 1, 1)
+    assert _lib.load().diagpu_spgemm_full_choice(n, na, nb, na + nb - 1, na * nb, C.byref(sh),
+                                                 cplx) == full
+
+
 def test_full_argument_errors():
     f = C.c_void_p(0x1000)   # never dereferenced: validation fails first
     name = "diagpu_spgemm_numeric_full_f32"

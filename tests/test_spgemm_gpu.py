@@ -962,7 +962,7 @@ def test_band_mfma_refuses_wide_spans(dev):
 
 
 # The contiguous-band kernel against the gather, bit for bit: rows on the edges
-# of its 64-, 128- and 256-row blocks and of its form limits (20000, 65536),
+# of its 64-, 128- and 256-row blocks and of a form limit (65536),
 # bands on both sides of its tiles of 4, 6 and 8 diagonals, wider than they
 # are high, off the main diagonal, and as wide as n; the largest A it takes.
 FULL_SHAPES = [
@@ -971,6 +971,16 @@ FULL_SHAPES = [
     (9999, -34, 69, -3, 7), (20000, -16, 33, -16, 33), (20011, 7, 20, -25, 9),
     (20161, -4, 8, -4, 9), (65536, -16, 33, -16, 33), (65537, -7, 15, -8, 17),
     (65791, -8, 30, -20, 40), (100000, -3, 7, -24, 49),
+]
+
+
+# The limits of the forms above 64-row blocks: 16384, 20000 and 32768 rows with
+# C diagonals on both sides of 24, 32, 52 and 64.
+FULL_SHAPES += [
+    (16384, -9, 19, -24, 49), (16385, -9, 19, -24, 49), (16385, -16, 33, -9, 20),
+    (16385, -16, 33, -9, 21), (16385, -8, 16, -8, 17), (16385, -8, 17, -8, 17),
+    (19999, -5, 11, -10, 22), (20000, -6, 12, -6, 13), (20000, -6, 13, -6, 13),
+    (32768, -12, 24, -20, 41), (32768, -12, 25, -20, 41), (32769, -12, 24, -20, 41),
 ]
 
 
