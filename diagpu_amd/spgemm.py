@@ -120,7 +120,7 @@ class SpgemmPlan:
         self._rstat = C.c_int32(0)
         self.shape = _lib.SpgemmShape()
         self._full, self._auto = {}, {}
-        self._written = None
+        self._written, self._versioned = None, not self._buf.is_inference()
         self._sym_fn = _lib.load().diagpu_spgemm_symbolic_shape
         self._sym_args, self._sym_caps, self._sym_ops = None, None, ()
         self.symbolic()
@@ -191,8 +191,8 @@ class SpgemmPlan:
         """What tells whether the caller has written plan arrays or counts since
         symbolic(): torch's count of writes to the buffer that the arrays are
         views of (inference tensors keep none), and the counts."""
-        buf, inf = self._buf, self.info
-        return (0 if buf.is_inference() else buf._version, inf.c_ndiag, inf.n_pairs)
+        inf = self.info
+        return (self._buf._version if self._versioned else 0, inf.c_ndiag, inf.n_pairs)
 
     # structure views (device tensors) --------------------------------------
     def c_offsets(self) -> torch.Tensor:
@@ -367,7 +367,7 @@ class SpgemmPlan:
         entries): it then stands in for the kernel that kernel_for names.  Not
         for a plan whose arrays or counts the caller has changed: that kernel
         reads no entries."""
-        if self._state() != self._written:
+        if not self.shape.contiguous or self._state() != self._written:
             return False
         v = self._full.get(dtype)
         if v is None:
@@ -390,12 +390,12 @@ class SpgemmPlan:
 
     def _auto_kernel(self, dtype) -> str:
         """The kernel "auto" runs, kept while nothing it depends on changes."""
-        state = lambda: (self._state(), self._astat is True, self._band is None)
+        state = self._state()
         kept = self._auto.get(dtype)
-        if kept is not None and kept[0] == state():
+        if kept is not None and kept[0] == (state, self._astat is True, self._band is None):
             return kept[1]
         kernel = "full" if self.uses_full(dtype) else self.kernel_for(dtype)
-        self._auto[dtype] = (state(), kernel)
+        self._auto[dtype] = ((state, self._astat is True, self._band is None), kernel)
         return kernel
 
     def numeric(self, A_vals: torch.Tensor, B_vals: torch.Tensor, C_vals: torch.Tensor,
