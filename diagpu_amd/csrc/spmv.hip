@@ -489,26 +489,42 @@ __global__ __launch_bounds__(64 * S) void spmv_split_kernel(
 }
 
 // Waves per tile of the split kernel, or 1 for the other kernels: a rule on
-// rows and diagonals alone, so that a real matrix takes the same order of
-// sums with real and with complex vectors.  About 8 diagonals per wave (4
-// at K <= 16, where the short kernel already issues every load at once).
-// Measured (us, 3 rotated sets, ring or short kernel -> split):
-//   fp32, K 64:  n = 1000 18.1 -> 5.4, 100003 17.5 -> 6.8, 300007 22.5 ->
-//                14.2, 600011 30.9 -> 26.8, 10^6 43.9 -> 43.7, 2 10^6 89.2
-//                -> 89.6
-//   fp64, K 64:  n = 100003 14.2 -> 11.8, 300007 30.7 -> 27.6, 10^6 88.6 ->
-//                92.3;  complex, K 85, n = 300007: 43.3 -> 41.8
-//   fp32 matrix, complex vector (half the rows per lane, so twice the
-//   waves): K 64, n = 300007 21.3 -> 20.6, 600011 35.8 -> 37.6
+// the matrix type, rows and diagonals alone, so that a real matrix takes the
+// same order of sums with real and with complex vectors.  About 8 diagonals
+// per wave (4 at K <= 16, where the short kernel already issues every load at
+// once).  Measured (us, 3 rotated sets, ring or short kernel -> split):
+//   fp32, K 64:  n = 1000 18.1 -> 5.4, 100003 17.5 -> 6.8, 250000 17.9 -> 13.2,
+//                399999 24.1 -> 20.7, 600011 30.9 -> 26.8, 10^6 43.9 -> 43.7
+//   fp64, K 64:  n = 130000 15.1 -> 14.4, 160000 20.9 -> 16.9, 210000 22.3 ->
+//                21.5, 250000 23.4 -> 25.0, 275000 30.4 -> 27.3, 350000 33.5 ->
+//                33.5, 399999 41.3 -> 39.3, 10^6 88.6 -> 92.3;  K 17: 90000 5.5
+//                -> 4.9, 130000 5.6 -> 5.7;  complex, K 85: 250000 29.9 -> 34.8,
+//                300000 41.8 -> 42.1
+//   fp32 matrix, complex vector: K 64, n = 250000 16.6 -> 18.3, 275000 21.2 ->
+//                19.8, 600011 35.8 -> 37.6
 //   fp32, K 16:  n = 50000 5.3 -> 4.0, 100003 5.3 -> 4.1;  fp64 50000 4.6 ->
-//                3.9, 100003 4.9 -> 4.9;  K 12: fp32 50000 4.6 -> 4.0
-// so the split ends where the last of the four types stops gaining: 400000
-// rows, and 100000 rows for K <= 16.
-inline int split_waves(int32_t rows, int K)
+//                3.9, 80000 0.97 of the rate, 99999 0.88;  K 12: fp32 50000 4.6
+//                -> 4.0
+// So it ends at 400000 rows, and 100000 (8-byte values 65536) for K <= 16.
+// With 8-byte values between, the ring kernel has one workgroup per 512 rows
+// and is the faster one where its last round of workgroups is well filled:
+// above 60 % of the 256 CUs.  (The fp32 matrix with a complex vector would end
+// there too, 0.8 to 1.0 of the ring's rate in those ranges; the real vector,
+// whose order of sums it shares, gains 1.1 to 1.4 there.)  It is the
+// faster one above 100000 rows, too, where a wave has 5 diagonals, which are
+// padded to 6 (fp64, K 40: 130000 0.91 of its rate, 300000 21.4 -> 23.9).
+template <typename TV, typename TX> int split_waves(int32_t rows, int K)
 {
-    if (rows <= 100000 && K >= 10 && K <= kShortMax) return K < 13 ? 2 : 4;
-    if (rows <= 400000 && K > kShortMax) return K < 20 ? 2 : (K < 40 ? 4 : 8);
-    return 1;
+    constexpr bool kWide = sizeof(TV) == 8;
+    if (K < 10) return 1;
+    if (K <= kShortMax) return rows <= (kWide ? 65536 : 100000) ? (K < 13 ? 2 : 4) : 1;
+    if (rows > 400000) return 1;
+    if (kWide) {
+        const int wgs = ceil_div<int>(rows, kBlock * Shape<TV, TX>::R), last = wgs % 256;
+        if (wgs <= 256 ? K < 20 && wgs > 195 : last == 0 || last > 154) return 1;
+        if (wgs > 195 && K >= 40 && K < 44) return 1;
+    }
+    return K < 20 ? 2 : (K < 40 ? 4 : 8);
 }
 
 template <typename TV, typename TX>
@@ -572,7 +588,7 @@ int spmv_run(int32_t rows, int32_t cols, int32_t num_diags, const int32_t* offs,
         return fail(DIAGPU_ERR_ARG, "%s: the dot epilogue needs x_size >= rows and its buffers",
                     name);
     if (lim == 0) K = 0;   // no column in range: y = 0 without touching values or x
-    const int S = dot || lim < Shape<TV, TX>::R ? 1 : split_waves(rows, K);
+    const int S = dot || lim < Shape<TV, TX>::R ? 1 : split_waves<TV, TX>(rows, K);
     if (S > 1) {
         const int32_t st = (int32_t)ceil_div<int64_t>(rows, 64 * Shape<TV, TX>::R);
         const int32_t sx = ceil_div<int32_t>(st, kNumXcd);

@@ -106,7 +106,8 @@ def test_poisson_closed_form_full_size(dev, dtype):
 
 # The kernel whose waves share a tile and split its diagonals: K on both sides
 # of each number of waves (10, 13, 17, 20, 40), of the chunks of 8 per wave
-# (64, 65, 129) and of its row limits (100000 for K <= 16, 400000), rows on
+# (64, 65, 129) and of its row limits (100000 and 65536 for K <= 16, 400000, and
+# for fp64 rounds of 256 workgroups of 512 rows: 99840, 209920, 262144), rows on
 # the edges of the 64-lane tiles (256 rows in fp32, 128 in fp64), offsets in
 # random order that leave the matrix on both sides, and an x shorter than the
 # rows reach.  No element outside [0, min(cols, len(x))) may be used: x and
@@ -115,7 +116,10 @@ def test_poisson_closed_form_full_size(dev, dtype):
 @pytest.mark.parametrize("rows,K", [(1, 10), (63, 12), (255, 13), (256, 16), (257, 17),
                                     (1000, 19), (1025, 20), (5000, 39), (5000, 40), (8191, 64),
                                     (8193, 65), (20000, 129), (100000, 16), (100001, 16),
-                                    (100003, 64), (400000, 17), (400001, 17)])
+                                    (100003, 64), (400000, 17), (400001, 17),
+                                    (65536, 13), (65537, 13), (99840, 19), (99841, 19),
+                                    (99841, 20), (131073, 27), (209920, 33), (209921, 33),
+                                    (262144, 44), (262145, 44), (99840, 43), (99841, 43)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_split_diagonals(dev, oracle, rows, K, dtype):
     rng = np.random.default_rng(rows + K)
