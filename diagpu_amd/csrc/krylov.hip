@@ -22,7 +22,7 @@
 // step j+1's d sum (sum_partials2): three launches per step.
 //
 // These are three launches a step for large n or many diagonals; few diagonals
-// up to kFusedRows rows run in one launch a step (k_lanczos_step), with the
+// up to 500000 rows run in one launch a step (k_lanczos_step), with the
 // same recurrence.  Which of the two is a rule on n, K and the workspace alone,
 // so equal calls give equal bits whatever else runs on the device.
 //
@@ -176,13 +176,14 @@ template <int BS> __device__ __forceinline__ void block_sum2(double& a, double& 
 // -> 335, 499849 432 -> 399; level with the three launches at 600000, and
 // slower above, where the columns' 16 runs a lane through the vector L1 cost
 // more than the launches (n = 2^22: 63 us a step against 53); so it ends at
-// kFusedRows.
+// kFusedRows.  7 diagonals, m = 20: n = 400000 294 -> 283 us, complex H 321 ->
+// 313, 450000 307 -> 325 and 337 -> 351: kFusedRowsWide.
 // The grid is at most kFusedWgs workgroups, each over tiles of 512 rows of its
 // XCD's range in step with the others, so that the next launch can add all
 // parts at its start in every workgroup.
 // ---------------------------------------------------------------------------
 constexpr int kFusedMax = 7;
-constexpr int kFusedRows = 500000;
+constexpr int kFusedRows = 500000, kFusedRowsWide = 400000;
 constexpr int kFusedWgs = 1024;
 
 // Scalars of step j (k_lanczos_update's) from the parts of d_j and q_{j-1}.
@@ -479,7 +480,8 @@ int expm_krylov(int32_t rows, int32_t cols, int32_t K, const int32_t* offs, cons
     const int stiles = spmv_tiles<TV, cf32>(rows);
 
     int st;
-    if (K >= 1 && K <= kFusedMax && rows <= kFusedRows && ws_bytes >= L.total) {
+    if (K >= 1 && K <= kFusedMax && rows <= (K > 5 ? kFusedRowsWide : kFusedRows) &&
+        ws_bytes >= L.total) {
         cf32* zbuf = reinterpret_cast<cf32*>(ws + L.zbuf);
         double* parts = reinterpret_cast<double*>(ws + L.parts);
         auto go = [&](auto km) {

@@ -143,7 +143,7 @@ DIAGPU_API int diagpu_expm_krylov_workspace_fused(int32_t n, int32_t m, size_t* 
  * H's action is used, Hermitian symmetry is the caller's promise), complex64
  * psi_0 and psi_t of n elements, 1 <= m <= 64 Lanczos steps.  Two kernels per
  * step (SpMV with a fused dot product, three-term update with a fused norm; up
- * to 7 diagonals and n = 500000, with a workspace of the _fused size: one
+ * to 5 diagonals and n = 500000 or 7 and 400000, with a workspace of the _fused size: one
  * kernel per step), deterministic fp64 reductions (the same call gives the
  * same bits, whatever runs beside it),
  * scalars kept on the device; one stream

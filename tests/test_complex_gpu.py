@@ -234,8 +234,8 @@ def test_propagator_pageable_readback(dev):
 
 # The fused-step and the three-launch propagators against exp(-i t H) psi_0 by a
 # Taylor series in complex128: numbers of diagonals on both sides of each fused
-# kernel's (3, 5, 7), rows on the edges of its tiles (512) and of its range
-# (500000), few rows and rows between, offsets that leave the
+# kernel's (3, 5, 7), rows on the edges of its tiles (512) and of its ranges
+# (500000, and 400000 above 5 diagonals), few rows and rows between, offsets that leave the
 # matrix altogether, m = 1 and 2.  |t| ||H|| <= 1, where m = 12 steps leave a
 # truncation below 1e-9; fp32 Lanczos vectors bound the rest: 12 steps of a few
 # units of 2^-24 each, well inside 2e-6.
@@ -243,7 +243,8 @@ def test_propagator_pageable_readback(dev):
     (5, [0, 1]), (256, [0, 255]), (257, [0, 1, 16]), (4097, [0, 1, 2, 64]), (16384, [1]),
     (16385, [0, 1, 2, 3, 100]), (131072, [0, 5]), (131073, [0, 1, 300]),
     (262144, [0, 1, 512, 513]), (262145, [0, 1, 512]), (262200, [0, 1, 512, 513]),
-    (300007, [0, 1, 2, 512, 700]), (500000, [0, 1]), (500001, [0, 707])])
+    (300007, [0, 1, 2, 512, 700]), (400000, [0, 1, 512, 700]), (400001, [0, 1, 512, 700]),
+    (500000, [0, 1]), (500001, [0, 707])])
 @pytest.mark.parametrize("complex_values", [True, False])
 def test_propagator_launch_forms(dev, n, pos, complex_values):
     g = torch.Generator(device=dev).manual_seed(n)
