@@ -246,19 +246,52 @@ def _narrow_first(X: HM) -> bool:
     return X.values.dtype == torch.float32 or X.ndiag <= _lib.ASTAT_MAX_A_C64
 
 
-class _HostPlans:
-    """The products C_t = H C_{t-1}, t = 1 .. steps, C_0 on the diagonals
-    `first`, planned on the host in one call (diagpu_chain_plans) and copied
-    to the device together: no read-back between the products.  `ok` is False
-    where a product is not the A-stationary kernel's (then the device plans
-    its products)."""
+# Plan entries per step up to which a chain's plans are formed on the host: 10
+# ns an entry there, against a launch, a kernel and a read-back for each plan on
+# the device.  H^3 of random offsets, n = 5000 to 37000, us a call, device / host:
+# 3828 entries 323 / 220, 5280 251 / 224, 6768 261 / 265, 10944 259 / 277, 18040
+# 297 / 355.
+HOST_PLAN_ENTRIES = 6144
 
-    def __init__(self, H: HM, first: list[int], steps: int):
+
+def _plan_entries(sizes: list[int], steps: int, reach: int) -> float:
+    """Entries of H C_{t-1}, t = 1 .. steps, where H, S and H S have `sizes`
+    diagonals (C_0 = H S) and C_t's lie within (t + 2) `reach`: exact for the
+    first, then with |C_t| about 3/4 |C_{t-1}|^2 / |C_{t-2}| (over
+    two steps to a fifth, over four to a half, on random sets and lattices)."""
+    h, s, c = sizes
+    total = 0.0
+    for t in range(1, steps + 1):
+        total += h * c
+        s, c = c, min(0.75 * c * c / max(s, 1), (t + 2) * reach + 1)
+    return total
+
+
+class _HostPlans:
+    """The products C_t = H C_{t-1}, t = 1 .. steps, C_0 = H S for S on the
+    diagonals `so`, planned on the host in one call (diagpu_chain_plans) and
+    copied to the device together: no read-back between the products.  `ok`
+    is False where a product is not the A-stationary kernel's, or the device
+    is the faster planner (then it plans the products)."""
+
+    def __init__(self, H: HM, so: list[int], steps: int):
         self.H, self.n = H, H.n
         ho = _host_offsets(H)
         dt = H.values.dtype
         cap = _lib.ASTAT_MAX_A if dt == torch.float32 else _lib.ASTAT_MAX_A_C64
-        self.ok = 4096 <= H.n < 1 << 30 and 1 <= len(ho) <= cap and len(first) > 0
+        self.ok = 4096 <= H.n < 1 << 30 and 1 <= len(ho) <= cap and len(so) > 0
+        self.first = None                       # C_0's offsets, once formed
+        if not self.ok:
+            return
+        nh, reach = len(ho), max(max(ho) - min(ho), max(so) - min(so))
+        # H S has at most half the sums where S is H (they come in pairs): a
+        # chain far beyond the limit is told without forming them
+        if min(nh * (len(so) + 1) // 2, 2 * reach + 1) * nh > 2 * HOST_PLAN_ENTRIES * steps:
+            self.ok = False
+            return
+        first = self.first = _sumset(self.n, ho, so)
+        self.ok = 0 < _plan_entries([nh, len(so), len(first)], steps,
+                                    reach) <= HOST_PLAN_ENTRIES * steps
         if not self.ok:
             return
         ha, sa = np.asarray(ho, np.int32), np.asarray(first, np.int32)
@@ -379,10 +412,10 @@ def _power_steps(H: HM, k: int) -> HM:
     complete once its symbolic phase has returned.  Products stay on the
     caller's stream, in order."""
     main = torch.cuda.current_stream(H.values.device)
-    plans = None
+    plans = first = None
     if k >= 3 and _narrow_first(H):
-        ho = _host_offsets(H)
-        plans = _HostPlans(H, _sumset(H.n, ho, ho), k - 2)
+        plans = _HostPlans(H, _host_offsets(H), k - 2)
+        first = plans.first
         if not plans.ok:
             plans = None
     side = _side_stream(H.values.device)
@@ -405,14 +438,14 @@ def _power_steps(H: HM, k: int) -> HM:
             else:
                 plan.numeric(P.values, H.values, C.values)
         if plans is not None and check.differ(H):   # while the product runs
-            plans = None
+            plans = first = None
         if plans is not None:
             v = C.values
             for t in range(1, k - 1):
                 v = plans.product(t, v)
             return plans.result(v)
-        C.host_offsets = _sumset(H.n, _host_offsets(H), _host_offsets(P))   # while it runs
-        P = C
+        C.host_offsets = first or _sumset(H.n, _host_offsets(H), _host_offsets(P))   # while it runs
+        P, first = C, None
     return P
 
 
@@ -574,9 +607,10 @@ def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event,
     side = _side_stream(H.values.device)
     # the steps after the first, planned on the host where they are all fused
     # products with I on their main diagonals
-    plans = None
+    plans = first = None
     if host_plans and order >= 3 and _narrow_first(H):
-        plans = _HostPlans(H, _sumset(H.n, _host_offsets(H), _host_offsets(S)), order - 2)
+        plans = _HostPlans(H, _host_offsets(S), order - 2)
+        first = plans.first
         if not (plans.ok and all(s.has_main for s in plans.steps)):
             plans = None
     if S.offsets is H.offsets and S.starts is H.starts and S.lengths is H.lengths:
@@ -614,7 +648,8 @@ def _taylor_steps(H: HM, t, order: int, S: HM, ready: torch.cuda.Event,
             for t_ in range(1, order - 1):
                 v = plans.product(t_, v, t / (order - 1 - t_), 1.0)
             return plans.result(v)
-        C.host_offsets = _sumset(H.n, _host_offsets(H), _host_offsets(S))   # while the product runs
+        C.host_offsets = first or _sumset(H.n, _host_offsets(H), _host_offsets(S))   # while it runs
+        first = None
         S = C if sigma else add_identity(C)
         if S.offsets is not C.offsets:
             side.wait_stream(main)              # a new structure, written on main

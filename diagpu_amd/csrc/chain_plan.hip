@@ -24,9 +24,12 @@
 namespace diagpu {
 namespace {
 
-// Plan entries of all steps together up to which the host forms them (0.1 ms
-// or so); beyond, the device's kernels are the faster planner.
+// Plan entries of all steps together up to which the host forms them (10 ns
+// an entry; callers that want the faster planner stop earlier).
 constexpr int64_t kMaxEntries = 32768;
+// Words of 64 offsets that a bit per offset may take (512 KiB); sums over a
+// wider span are sorted.
+constexpr int64_t kSpanWords = 1 << 16;
 
 int64_t absl(int64_t x) { return x < 0 ? -x : x; }
 int64_t min0(int64_t x) { return x < 0 ? x : 0; }
@@ -59,51 +62,95 @@ int chain_plans(const char* fn, int32_t n, int32_t nh, const int32_t* h, int32_t
                 const int32_t* s0, int32_t steps, char* out, size_t capacity, size_t* needed,
                 diagpu_chain_step* info)
 {
-    std::vector<int32_t> b(s0, s0 + ns), c;
+    std::vector<std::vector<int32_t>> lists((size_t)steps + 1);   // C_t's offsets
+    std::vector<uint64_t> bits;
+    std::vector<int32_t> before, rank;
     std::vector<int64_t> bstart, count;
-    std::vector<int32_t> next((size_t)nh);
-    size_t at = 0;
+    // The sums of step t lie in [low(t), high(t)], inside (-n, n).
+    auto low = [&](int32_t t) {
+        const auto& b = lists[(size_t)t];
+        return b.empty() ? 0 : std::max<int64_t>((int64_t)h[0] + b.front(), 1 - (int64_t)n);
+    };
+    auto high = [&](int32_t t) {
+        const auto& b = lists[(size_t)t];
+        return b.empty() ? -1
+                         : std::min<int64_t>((int64_t)h[nh - 1] + b.back(), (int64_t)n - 1);
+    };
+    // All offsets first (a bit per offset of the span, 1 to 2 ns a sum), so
+    // that a chain that is refused costs little.
+    lists[0].assign(s0, s0 + ns);
     int64_t entries = 0;
     for (int32_t t = 0; t < steps; ++t) {
-        const int32_t nb = (int32_t)b.size();
-        entries += (int64_t)nh * nb;
+        const std::vector<int32_t>& b = lists[(size_t)t];
+        std::vector<int32_t>& c = lists[(size_t)t + 1];
+        entries += (int64_t)nh * (int64_t)b.size();
         if (entries > kMaxEntries)
             return fail(DIAGPU_ERR_OVERFLOW, "%s: more than %lld entries by step %d", fn,
                         (long long)kMaxEntries, t + 1);
+        const int64_t lo = low(t), span = high(t) - lo + 1;
+        const int64_t words = span <= 0 ? 0 : (span + 63) / 64;
+        if (words > kSpanWords) {
+            for (int32_t a = 0; a < nh; ++a)
+                for (const int32_t db : b) {
+                    const int64_t q = (int64_t)h[a] + db - lo;
+                    if (q >= 0 && q < span) c.push_back((int32_t)(q + lo));
+                }
+            std::sort(c.begin(), c.end());
+            c.erase(std::unique(c.begin(), c.end()), c.end());
+            continue;
+        }
+        bits.assign((size_t)words, 0);
+        for (int32_t a = 0; a < nh; ++a)
+            for (const int32_t db : b) {
+                const int64_t q = (int64_t)h[a] + db - lo;
+                if (q >= 0 && q < span) bits[(size_t)(q >> 6)] |= 1ull << (q & 63);
+            }
+        for (int64_t w = 0; w < words; ++w)
+            for (uint64_t m = bits[(size_t)w]; m; m &= m - 1)
+                c.push_back((int32_t)(lo + 64 * w + __builtin_ctzll(m)));
+    }
+    size_t at = 0;
+    for (int32_t t = 0; t < steps; ++t) {
+        const std::vector<int32_t>&b = lists[(size_t)t], &c = lists[(size_t)t + 1];
+        const int32_t nb = (int32_t)b.size();
         bstart.resize((size_t)nb);
         int64_t bnnz = 0;
         for (int32_t i = 0; i < nb; ++i) {
             bstart[i] = bnnz;
             bnnz += n - absl(b[i]);
         }
-        // C offsets: the nh ascending lists h[a] + b[.], merged
-        c.clear();
-        std::fill(next.begin(), next.end(), 0);
-        for (;;) {
-            int64_t lo = INT64_MAX;
-            for (int32_t a = 0; a < nh; ++a)
-                if (next[a] < nb) lo = std::min<int64_t>(lo, (int64_t)h[a] + b[next[a]]);
-            if (lo == INT64_MAX) break;
-            for (int32_t a = 0; a < nh; ++a)
-                if (next[a] < nb && (int64_t)h[a] + b[next[a]] == lo) ++next[a];
-            if (lo > -(int64_t)n && lo < n) c.push_back((int32_t)lo);
+        // C's bits again, and the offsets before each word
+        const int64_t lo = low(t), span = high(t) - lo + 1;
+        const bool marked = span <= 64 * kSpanWords;
+        const size_t words = span <= 0 || !marked ? 0 : (size_t)((span + 63) / 64);
+        bits.assign(words, 0);
+        if (marked)
+            for (const int32_t dc : c) bits[(size_t)((dc - lo) >> 6)] |= 1ull << ((dc - lo) & 63);
+        before.resize(words);
+        int32_t seen = 0;
+        for (size_t w = 0; w < words; ++w) {
+            before[w] = seen;
+            seen += __builtin_popcountll(bits[w]);
         }
         diagpu_chain_step& s = info[t];
         s = diagpu_chain_step{};
         s.c_ndiag = (int64_t)c.size();
         s.b_extent = bnnz;
-        // entries per C diagonal: for each a, its sums in ascending order
+        // each sum's C diagonal, in B order, and the entries per C diagonal
         count.assign(c.size() + 1, 0);
-        for (int32_t a = 0; a < nh; ++a) {
-            size_t k = 0;
-            for (int32_t i = 0; i < nb; ++i) {
-                const int64_t dc = (int64_t)h[a] + b[i];
-                if (dc <= -(int64_t)n) continue;
-                if (dc >= n) break;
-                while (c[k] < dc) ++k;
-                ++count[k + 1];
+        rank.resize((size_t)nh * nb);
+        for (int32_t i = 0; i < nb; ++i)
+            for (int32_t a = 0; a < nh; ++a) {
+                const int64_t q = (int64_t)h[a] + b[i] - lo;
+                int32_t k = -1;
+                if (q >= 0 && q < span) {
+                    const size_t w = (size_t)(q >> 6);
+                    k = marked ? before[w] + __builtin_popcountll(bits[w] & ((1ull << (q & 63)) - 1))
+                               : (int32_t)(std::lower_bound(c.begin(), c.end(), q + lo) - c.begin());
+                    ++count[(size_t)k + 1];
+                }
+                rank[(size_t)i * nh + a] = k;
             }
-        }
         for (size_t k = 0; k < c.size(); ++k) {
             s.c_nnz += n - absl(c[k]);
             s.max_pairs = std::max(s.max_pairs, count[k + 1]);
@@ -129,13 +176,11 @@ int chain_plans(const char* fn, int32_t n, int32_t nh, const int32_t* h, int32_t
                 count[k + 1] = ptr[k];   // the diagonal's next free entry
             }
             ptr[c.size()] = g;
-            std::fill(next.begin(), next.end(), 0);   // each a's place in c
-            for (int32_t i = 0; i < nb; ++i)          // B order within a C diagonal
+            for (int32_t i = 0; i < nb; ++i)   // B order within a C diagonal
                 for (int32_t a = 0; a < nh; ++a) {
+                    const int32_t k = rank[(size_t)i * nh + a];
+                    if (k < 0) continue;
                     const int64_t da = h[a], db = b[i], dc = da + db;
-                    if (dc <= -(int64_t)n || dc >= n) continue;
-                    int32_t& k = next[a];
-                    while (c[k] < dc) ++k;
                     // GPair {A start, B start, ash, bsh, al, bl} as a record
                     const int64_t ash = min0(da) - min0(dc), bsh = da + min0(db) - min0(dc);
                     const int64_t lo = std::max<int64_t>(0, std::max(-ash, -bsh));
@@ -155,7 +200,6 @@ int chain_plans(const char* fn, int32_t n, int32_t nh, const int32_t* h, int32_t
             tail[3] = h[nh - 1];
         }
         at = end;
-        b.swap(c);
     }
     *needed = at;
     if (at > capacity)

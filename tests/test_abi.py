@@ -389,7 +389,8 @@ def test_chain_plans_argument_errors():
     (10, [0], [0], 3), (10, [-9, 9], [-9, 9], 2), (50, [-7, -1, 0, 1, 7], [-7, 0, 3], 4),
     (40, [-13, 2, 5], [-39, -20, 0, 38], 5), (9, [-3, 1, 4], [-8, -2, 0, 5, 8], 6),
     (5000, [-300, -17, -1, 0, 1, 17, 300], [-300, -17, -1, 0, 1, 17, 300], 4),
-    (100000, [5, 90000], [-99999, -5, 7], 3)])
+    (100000, [5, 90000], [-99999, -5, 7], 3),
+    (5000000, [-4000000, -3, 0, 5, 900000], [-2500000, 0, 7, 3000000], 3)])
 def test_chain_plans_match_the_reference_planners(oracle, n, h, s, steps):
     """Every array against the oracle's restatement of the reference planners:
     C structure, pair_ptr, and each record against its GPair (A index, range
