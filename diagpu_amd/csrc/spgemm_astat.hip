@@ -649,18 +649,26 @@ int launch_rows(const char* fn, int32_t n, const int32_t* A_off, const int64_t* 
     // noise but one (128 x 16 at 2^20, 6%).  Lost with it: complex values at
     // 2 rows per lane (config 5 complex, 8 rounds: 6.13 -> 6.28 ms at G = 2)
     // and the 8 rows per lane of the Taylor chain's products (numeric 1.96 ->
-    // 2.05 ms).  Complex values at 4 rows per lane take G = 2 from 100 C
-    // diagonals up to 3 rounds (us, G = 1 -> 2): 5 x 120 and 9 x 100 random
-    // diagonals at n = 150000 185 -> 150 and 242 -> 197, 36 x 60 492 -> 449;
-    // the 7-point stencil times its 63 and 129 diagonals at n = 151951 60.0 ->
-    // 55.4 and 122 -> 105.  Above that 2 % either way (604800: 306 -> 317, 10^6
-    // 541 -> 529), and it loses on short lists (25 C diagonals at 10^6: 49 ->
-    // 66, 63 at 604800: 83.5 -> 85.8).
+    // 2.05 ms).  Complex values at 4 rows per lane take G = 2 for at most 14 A
+    // diagonals from 100 C diagonals, up to 3 rounds whose last is up to a
+    // quarter full, or a half to three quarters (2 whole / slots then just
+    // passes a whole number: half-size workgroups end half a round earlier).
+    // Rate of G = 2 over G = 1, geometric mean over 13 to 18 products (random
+    // 5 x 30 to 14 x 23, bands, the 7-point stencil's chain): 1.16 at n =
+    // 132000 (1.01 rounds), 1.12 at 138000, 1.08 at 150000, 1.04 at 163000,
+    // 1.04 at 200000 and 210000, 1.03 at 225000 and 275000; the stencil times
+    // its 63 and 129 diagonals at n = 151951 60.0 -> 55.4 us and 122 -> 105.
+    // Between these: 0.97 at 131000 (1.00 rounds), 0.98 at 170000 and 190000,
+    // 0.99 at 236000 and 245000, 0.90 to 1.05 at 300000.  It loses where two
+    // workgroups stage more A diagonals (16 x 40 0.94 at 200000 to 245000, 36
+    // x 12 0.88 at 251000, 71 x 3 0.88), is level above 3 rounds (604800: 306
+    // -> 317 us, 10^6 541 -> 529), and loses on short lists (25 C diagonals at
+    // 10^6: 49 -> 66, 63 at 604800: 83.5 -> 85.8).
     int64_t G = 1;
-    if constexpr (sizeof(T) == 8 && R == 4)
-        if (c_ndiag >= 100 &&
-            ceil_div<int64_t>(ceil_div<int64_t>((int64_t)n + kLead, kRB), slots) <= 3)
-            G = 2;
+    if constexpr (sizeof(T) == 8 && R == 4) {
+        const int64_t whole = ceil_div<int64_t>((int64_t)n + kLead, kRB), half = 2 * whole % slots;
+        if (nA <= 14 && c_ndiag >= 100 && whole <= 3 * slots && half && 2 * half <= slots) G = 2;
+    }
     if constexpr (sizeof(T) == 4 && R == 4) {
         const int64_t r0 = ceil_div<int64_t>(ceil_div<int64_t>((int64_t)n + kLead, kRB), slots);
         while (G < 4 && r0 * G < 16 && c_ndiag >= 2 * G * kPrefetchDiagsPerWave * kWaves) G *= 2;

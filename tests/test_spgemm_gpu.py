@@ -1109,3 +1109,22 @@ def test_astat_launch_shapes_same_bits(dev, n, nx, ny, k, dtype):
     C = torch.full((plan.info.c_nnz,), float("nan"), dtype=dtype, device=dev)
     plan.numeric(av, bv, C, kernel="astat")
     assert torch.equal(word(C), word(plan.multiply(av, bv, kernel="gather")))
+
+
+# Complex values over two workgroups per block: at most 14 A diagonals, 100 C
+# diagonals, and the last of at most 3 rounds of 512 blocks of 256 rows (16
+# rows of lead) up to a quarter full or a half to three quarters.  Both sides
+# of each limit, with the gather's bits.
+@pytest.mark.parametrize("n,na", [(131056, 14), (131057, 14), (131057, 15), (163824, 14),
+                                  (163825, 14), (196593, 5), (229360, 14), (229361, 9)])
+def test_astat_complex_split_limits_same_bits(dev, n, na):
+    A = workloads.hm_random(n, [37 * i - 90 for i in range(na)], seed=n, device=dev)
+    B = workloads.hm_random(n, [1000 * i - 9000 for i in range(21)], seed=na, device=dev)
+    av = torch.complex(A.values, torch.roll(A.values, 3)).contiguous()
+    bv = torch.complex(B.values, torch.roll(B.values, 5)).contiguous()
+    plan = SpgemmPlan(A, B)
+    assert plan.info.c_ndiag >= 100 and plan.kernel_for(torch.complex64) == "astat"
+    C = torch.full((plan.info.c_nnz,), float("nan"), dtype=torch.complex64, device=dev)
+    plan.numeric(av, bv, C, kernel="astat")
+    assert torch.equal(torch.view_as_real(C).view(torch.int32),
+                       torch.view_as_real(plan.multiply(av, bv, kernel="gather")).view(torch.int32))
