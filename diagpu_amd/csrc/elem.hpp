@@ -61,6 +61,11 @@ template <typename T> __device__ __forceinline__ T zero_of();
 template <> __device__ __forceinline__ float zero_of<float>() { return 0.f; }
 template <> __device__ __forceinline__ double zero_of<double>() { return 0.0; }
 template <> __device__ __forceinline__ cf32 zero_of<cf32>() { return cf32{0.f, 0.f}; }
+// -0: the value that leaves every other (either zero too) as it is when added
+template <typename T> __device__ __forceinline__ T neg_zero_of();
+template <> __device__ __forceinline__ float neg_zero_of<float>() { return -0.f; }
+template <> __device__ __forceinline__ double neg_zero_of<double>() { return -0.0; }
+template <> __device__ __forceinline__ cf32 neg_zero_of<cf32>() { return cf32{-0.f, -0.f}; }
 
 // Re(conj(u) * y) in fp64
 __device__ __forceinline__ double dotpart(float u, float y) { return (double)u * (double)y; }

@@ -135,13 +135,22 @@ enum EdgeMode {
 // clamped to [0, gn) so all loads are valid, and the slots past the end are
 // masked.  kEdgeRun needs lim >= R and masks every term whose column is
 // outside [0, lim).
-template <typename TV, typename TX, int W, int MODE>
+// With LG > 0 the diagonals [gn w / S, gn (w + 1) / S), S = 2^LG, make one sum
+// each, and these are added in order of w: the split kernel's sums, bit for
+// bit (the first is added to -0, which leaves it as it is).
+template <typename TV, typename TX, int W, int MODE, int LG = 0>
 __device__ __forceinline__ void ring_group(int64_t r, int64_t cols, int64_t lim, int gn,
                                            const int32_t* __restrict__ offs,
                                            const TV* __restrict__ vg, const TX* __restrict__ x,
                                            Run<TX, Shape<TV, TX>::R>& acc)
 {
     constexpr int R = Shape<TV, TX>::R;
+    Run<TX, R> sum;
+    int w = 1, next = gn >> LG;   // next: sum w's first diagonal
+    if constexpr (LG > 0) {
+#pragma unroll
+        for (int e = 0; e < R; ++e) sum.v[e] = neg_zero_of<TX>();
+    }
     Run<TV, R> a[W];
     Run<TX, R> b[W];
     // a run start clamped to a valid run, [0, lim - R] (kEdgeRun)
@@ -163,6 +172,16 @@ __device__ __forceinline__ void ring_group(int64_t r, int64_t cols, int64_t lim,
     };
     // slot j holds diagonal k (k uniform); `on` = the slot is part of the group
     auto consume = [&](int j, int k, bool on) {
+        if constexpr (LG > 0) {
+            const bool ends = on && k == next;   // sum w - 1 is complete
+#pragma unroll
+            for (int e = 0; e < R; ++e) {
+                sum.v[e] = sel(ends, add_(sum.v[e], acc.v[e]), sum.v[e]);
+                acc.v[e] = sel(ends, zero_of<TX>(), acc.v[e]);
+            }
+            w += ends;
+            next = (int)((int64_t)gn * w >> LG);
+        }
         if constexpr (MODE == kInterior) {
 #pragma unroll
             for (int e = 0; e < R; ++e)
@@ -217,17 +236,21 @@ __device__ __forceinline__ void ring_group(int64_t r, int64_t cols, int64_t lim,
         const int kc = k0 + W + j;
         consume(j, kc < gn ? kc : gn - 1, kc < gn);
     }
+    if constexpr (LG > 0) {
+#pragma unroll
+        for (int e = 0; e < R; ++e) acc.v[e] = add_(sum.v[e], acc.v[e]);
+    }
 }
 
 // A non-interior tile (lim >= R: the host sends narrower matrices to
 // spmv_narrow_kernel).
-template <typename TV, typename TX>
+template <typename TV, typename TX, int LG = 0>
 __device__ __forceinline__ void edge_group(int64_t r, int64_t cols, int64_t lim, int gn,
                                            const int32_t* __restrict__ offs,
                                            const TV* __restrict__ vg, const TX* __restrict__ x,
                                            Run<TX, Shape<TV, TX>::R>& acc)
 {
-    ring_group<TV, TX, Shape<TV, TX>::WR, kEdgeRun>(r, cols, lim, gn, offs, vg, x, acc);
+    ring_group<TV, TX, Shape<TV, TX>::WR, kEdgeRun, LG>(r, cols, lim, gn, offs, vg, x, acc);
 }
 
 template <typename TX, int R>
@@ -267,8 +290,8 @@ __device__ __forceinline__ void dot_epilogue(const Run<TX, R>& acc, const TX* __
 // Kernels
 // ---------------------------------------------------------------------------
 
-// K > kShortMax: one ring over all K diagonals.
-template <typename TV, typename TX, bool DOT>
+// K > kShortMax: one ring over all K diagonals (LG: ring_group).
+template <typename TV, typename TX, bool DOT, int LG = 0>
 __global__ __launch_bounds__(kBlock) void spmv_ring_kernel(
     int32_t rows, int32_t cols, int64_t lim, int32_t K, const int32_t* __restrict__ offs,
     const TV* __restrict__ vals, const TX* __restrict__ x, TX* __restrict__ y, int32_t tiles,
@@ -298,9 +321,9 @@ __global__ __launch_bounds__(kBlock) void spmv_ring_kernel(
 #pragma unroll
     for (int e = 0; e < R; ++e) acc.v[e] = zero_of<TX>();
     if (interior)
-        ring_group<TV, TX, S::W, kInterior>(r, cols, lim, K, offs, vals, x, acc);
+        ring_group<TV, TX, S::W, kInterior, LG>(r, cols, lim, K, offs, vals, x, acc);
     else
-        edge_group<TV, TX>(r, cols, lim, K, offs, vals, x, acc);
+        edge_group<TV, TX, LG>(r, cols, lim, K, offs, vals, x, acc);
     store_rows<TX, R>(y, r, rows, acc, interior);
     if constexpr (DOT) dot_epilogue<TX, R>(acc, x, r, rows, interior, tile, tiles, da);
 }
@@ -508,9 +531,9 @@ __global__ __launch_bounds__(64 * S) void spmv_split_kernel(
 // So it ends at 400000 rows, and 100000 (8-byte values 65536) for K <= 16.
 // With 8-byte values between, the ring kernel has one workgroup per 512 rows
 // and is the faster one where its last round of workgroups is well filled:
-// above 60 % of the 256 CUs.  (The fp32 matrix with a complex vector would end
-// there too, 0.8 to 1.0 of the ring's rate in those ranges; the real vector,
-// whose order of sums it shares, gains 1.1 to 1.4 there.)  It is the
+// above 60 % of the 256 CUs.  (The fp32 matrix with a complex vector, which
+// shares the real vector's order of sums, then forms them in the ring kernel:
+// ring_sums.)  It is the
 // faster one above 100000 rows, too, where a wave has 5 diagonals, which are
 // padded to 6 (fp64, K 40: 130000 0.91 of its rate, 300000 21.4 -> 23.9).
 template <typename TV, typename TX> int split_waves(int32_t rows, int K)
@@ -525,6 +548,25 @@ template <typename TV, typename TX> int split_waves(int32_t rows, int K)
         if (wgs > 195 && K >= 40 && K < 44) return 1;
     }
     return K < 20 ? 2 : (K < 40 ? 4 : 8);
+}
+
+// A real matrix with a complex vector takes twice the workgroups of a real
+// vector for the same rows, so the ring kernel fills the chip sooner: where
+// its last round of 256 workgroups is well filled it forms the split kernel's
+// sums (the real vector's order, for which the split kernel stays the faster)
+// at 0.95 to 1.0 of its rate with one sum.  Where a wave of the split kernel
+// would have 5 or 7 diagonals, padded to 6 or 8, it is the faster one earlier.
+// Rate against the split kernel (fp32 matrix): n = 262144 (2 full rounds) K =
+// 24 1.06, 28 1.23, 40 1.26, 64 1.11, 78 1.10, 96 0.97; 225000 (1.7 rounds) K =
+// 40 1.14, 64 0.99, 96 0.87; 150000 (1.1) 0.67 to 0.93; 392000 (3.0) K = 24
+// 1.02, 40 1.31, 78 1.09; 290000 (2.2) K = 28 1.02, 40 1.11, 78 0.89.
+template <typename TV, typename TX> bool ring_sums(int32_t rows, int K, int S)
+{
+    const int wgs = ceil_div<int>(rows, Shape<TV, TX>::TILE);
+    if (K <= kShortMax || wgs <= 256) return false;
+    const int last = (wgs - 1) % 256 + 1, per = K / S;
+    if (per == 5 || per == 7) return wgs > 512 || last > 128;
+    return last > (wgs > 512 ? 128 : 180);
 }
 
 template <typename TV, typename TX>
@@ -589,6 +631,19 @@ int spmv_run(int32_t rows, int32_t cols, int32_t num_diags, const int32_t* offs,
                     name);
     if (lim == 0) K = 0;   // no column in range: y = 0 without touching values or x
     const int S = dot || lim < Shape<TV, TX>::R ? 1 : split_waves<TV, TX>(rows, K);
+    const int32_t tiles = spmv_tiles<TV, TX>(rows);
+    const int32_t per_xcd = ceil_div<int32_t>(tiles, kNumXcd);
+    if constexpr (sizeof(TV) < sizeof(TX)) {
+        if (S > 1 && ring_sums<TV, TX>(rows, K, S)) {
+            hipLaunchKernelGGL((S == 2   ? spmv_ring_kernel<TV, TX, false, 1>
+                                : S == 4 ? spmv_ring_kernel<TV, TX, false, 2>
+                                         : spmv_ring_kernel<TV, TX, false, 3>),
+                               dim3(per_xcd * kNumXcd), dim3(kBlock), 0, as_stream(stream), rows,
+                               cols, lim, K, offs, vals, x, y, tiles, per_xcd,
+                               DotArgs{nullptr, nullptr});
+            return check_launch(name);
+        }
+    }
     if (S > 1) {
         const int32_t st = (int32_t)ceil_div<int64_t>(rows, 64 * Shape<TV, TX>::R);
         const int32_t sx = ceil_div<int32_t>(st, kNumXcd);
@@ -599,8 +654,6 @@ int spmv_run(int32_t rows, int32_t cols, int32_t num_diags, const int32_t* offs,
                            K, offs, vals, x, y, st, sx);
         return check_launch(name);
     }
-    const int32_t tiles = spmv_tiles<TV, TX>(rows);
-    const int32_t per_xcd = ceil_div<int32_t>(tiles, kNumXcd);
     const DotArgs da = dot ? *dot : DotArgs{nullptr, nullptr};
     hipLaunchKernelGGL((dot ? pick_kernel<TV, TX, true>(K, lim) : pick_kernel<TV, TX, false>(K, lim)),
                        dim3(per_xcd * kNumXcd), dim3(kBlock), 0, as_stream(stream), rows, cols,

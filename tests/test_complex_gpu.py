@@ -91,6 +91,34 @@ def test_real_matrix_complex_state_equals_real_kernel_per_part(dev, K):
     assert torch.equal(y.real, yr) and torch.equal(y.imag, yi)
 
 
+# A real matrix with a complex vector forms the real vector's sums in the ring
+# kernel from 131073 rows where that is the faster one, in two, four or eight
+# sums of even and uneven length: both sides of its limits (5 and 7 diagonals
+# per sum, rounds of 131072 rows), rows beyond the columns and a short x, bit
+# for bit the products with the real and the imaginary part.
+@pytest.mark.parametrize("rows,cols,xs,K", [
+    (262144, 262144, 262144, 17), (262144, 262144, 262144, 19), (223233, 223233, 223233, 24),
+    (223232, 223232, 223232, 24), (196609, 196609, 196609, 28), (196608, 196608, 196608, 28),
+    (262145, 262145, 262145, 41), (262144, 262100, 262100, 64), (262001, 262144, 261003, 78),
+    (399999, 399999, 399999, 97), (400000, 400000, 400000, 131), (327681, 327681, 327681, 39)])
+def test_mixed_sums_are_the_real_ones(dev, rows, cols, xs, K):
+    g = torch.Generator().manual_seed(rows + K)
+    half = [300, 2500][K % 2]
+    offs = (torch.randperm(2 * half + 1, generator=g)[:K] - half).to(torch.int32).to(dev)
+    vals = torch.randn(K * cols, generator=g)
+    vals[torch.rand(K * cols, generator=g) < 0.1] = 0.0
+    vals[7 * K] = float("inf")
+    x = torch.randn(xs, dtype=torch.complex64, generator=g).to(dev)
+    vals = vals.to(dev)
+    y = spmv_recon(offs, vals, rows, cols, x)
+    word = lambda v: v.contiguous().view(torch.int32)
+    for got, part in ((y.real, x.real), (y.imag, x.imag)):
+        want = spmv_recon(offs, vals, rows, cols, part.contiguous())
+        num = ~torch.isnan(want)
+        assert torch.equal(torch.isnan(got), ~num)
+        assert torch.equal(word(got)[num], word(want)[num])
+
+
 def test_complex_spmv_full_size_poisson(dev, oracle):
     """Benchmark config 2's stencil with complex values (i times the real
     stencil) and a complex state: y = i H x, checked over every row."""
