@@ -527,8 +527,10 @@ __global__ __launch_bounds__(64 * S) void spmv_split_kernel(
 //                19.8, 600011 35.8 -> 37.6
 //   fp32, K 16:  n = 50000 5.3 -> 4.0, 100003 5.3 -> 4.1;  fp64 50000 4.6 ->
 //                3.9, 80000 0.97 of the rate, 99999 0.88;  K 12: fp32 50000 4.6
-//                -> 4.0
-// So it ends at 400000 rows, and 100000 (8-byte values 65536) for K <= 16.
+//                -> 4.0;  K 10: n = 1000 fp32 3.59 -> 3.71, complex vector 2.78 ->
+//                3.09, 5000 1.00 to 1.04 of the rate, 15000 1.03 to 1.08
+// So it starts at K = 10, from 4096 rows (K = 12 below: K 12, n = 1000 1.06 to
+// 1.16), and ends at 400000 rows, and 100000 (8-byte values 65536) for K <= 16.
 // With 8-byte values between, the ring kernel has one workgroup per 512 rows
 // and is the faster one where its last round of workgroups is well filled:
 // above 60 % of the 256 CUs.  (The fp32 matrix with a complex vector, which
@@ -539,7 +541,7 @@ __global__ __launch_bounds__(64 * S) void spmv_split_kernel(
 template <typename TV, typename TX> int split_waves(int32_t rows, int K)
 {
     constexpr bool kWide = sizeof(TV) == 8;
-    if (K < 10) return 1;
+    if (K < 10 || (K < 12 && rows < 4096)) return 1;
     if (K <= kShortMax) return rows <= (kWide ? 65536 : 100000) ? (K < 13 ? 2 : 4) : 1;
     if (rows > 400000) return 1;
     if (kWide) {

@@ -108,7 +108,8 @@ def test_poisson_closed_form_full_size(dev, dtype):
 # of each number of waves (10, 13, 17, 20, 40), of the chunks of 8 per wave
 # (64, 65, 129) and of its row limits (100000 and 65536 for K <= 16, 400000, and
 # for fp64 rounds of 256 workgroups of 512 rows: 99840, 209920, 262144), rows on
-# the edges of the 64-lane tiles (256 rows in fp32, 128 in fp64), offsets in
+# the edges of the 64-lane tiles (256 rows in fp32, 128 in fp64), the 4096 rows
+# below which 10 and 11 diagonals are not split, offsets in
 # random order that leave the matrix on both sides, and an x shorter than the
 # rows reach.  No element outside [0, min(cols, len(x))) may be used: x and
 # the matrix are NaN there.  Any order of K <= 166 fp32 terms stays within the
@@ -119,7 +120,8 @@ def test_poisson_closed_form_full_size(dev, dtype):
                                     (100003, 64), (400000, 17), (400001, 17),
                                     (65536, 13), (65537, 13), (99840, 19), (99841, 19),
                                     (99841, 20), (131073, 27), (209920, 33), (209921, 33),
-                                    (262144, 44), (262145, 44), (99840, 43), (99841, 43)])
+                                    (262144, 44), (262145, 44), (99840, 43), (99841, 43),
+                                    (4095, 11), (4096, 11), (4095, 12), (4096, 10)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_split_diagonals(dev, oracle, rows, K, dtype):
     rng = np.random.default_rng(rows + K)
